@@ -47,6 +47,7 @@
 // ends with 4 consecutive rows of one column of C, which the epilogue
 // writes as two 16-byte stores.
 #include "common.hpp"
+#include "dgemm_dl.hpp"
 
 namespace cosma_amd {
 namespace {
@@ -423,210 +424,6 @@ __global__ __launch_bounds__(NT) void dgemm_mfma_kernel(
     gemm_tile<BM, BN, TA, TB, VEC>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, vec_c, m0, n0, sm);
 }
 
-// ------------------------------------ GEMM with direct global-to-LDS loads
-// M and N multiples of 128, K a multiple of 16, 16-byte aligned operands with
-// even leading dimensions; any transposes.  128 x 128 tiles at two
-// workgroups per CU (two waves per SIMD: 128 accumulator registers per
-// lane), so that one workgroup's barrier, fragment reads and load waits
-// overlap the other's MFMAs; the operand tiles go from global memory
-// straight into LDS (global_load_lds_dwordx4: lane l of a wave instruction
-// writes the 16 bytes at the instruction's LDS base + 16 l), with no
-// register staging.  LDS layouts per stage and operand:
-//   k-contiguous operand (A 'T', B 'N'): row r holds its eight k-pairs
-//     (128 bytes), pair kp in slot kp ^ (r & 7); the global addresses of the
-//     loads apply that permutation, so eight lanes still read one 128-byte
-//     row.  A fragment is one 16-byte read.
-//   row-contiguous operand (A 'N', B 'T'): k-row k holds the tile's 128 rows
-//     (one 1 KB wave load), k-rows RC_LD doubles apart (the 64-byte pad puts
-//     the four k-rows that one fragment read touches on alternate halves of
-//     the banks).  A fragment is two 8-byte reads (k = 2 kp and 2 kp + 1).
-// The fragments (lane g supplies the pair kp = 4 ks + g of its permuted
-// row), the MFMA order and the epilogue are gemm_tile's, so the results are
-// bit-identical to dgemm_mfma_kernel's.
-constexpr int DL_TILE = 128;
-constexpr int KC_SIZE = DL_TILE * BK;          // doubles of a k-contiguous operand tile
-constexpr int RC_LD = DL_TILE + 8;             // doubles between the k-rows of a row-contiguous tile
-constexpr int RC_SIZE = BK * RC_LD;
-// s_waitcnt immediate (gfx9 fields: vmcnt bits 3:0 and 15:14, expcnt 6:4,
-// lgkmcnt 11:8) waiting for vmcnt = 0 only; OR a count into bits 3:0.
-constexpr int WAIT_VMCNT0 = 0x0F70;
-
-__device__ __forceinline__ void lds_dma16(const double *g, double *lds) {
-    __builtin_amdgcn_global_load_lds(static_cast<const void *>(g),
-                                     (__attribute__((address_space(3))) void *)lds, 16, 0, 0);
-}
-
-// One operand tile in LDS: the loads of step k0 for wave `wave`, and the
-// fragment of (row r, k-pair kp).
-template <bool KCONTIG>
-struct DlOperand {
-    static constexpr int SIZE = KCONTIG ? KC_SIZE : RC_SIZE;
-    const double *p;   // this thread's load address for k0 = 0
-    int64_t ld;
-    __device__ __forceinline__ DlOperand(const double *x, int64_t ld_, int64_t r0) : ld(ld_) {
-        const int t = threadIdx.x, lane = t & 63;
-        if (KCONTIG) {
-            // slot q * 256 + t is row 32 q + t / 8, slot t % 8, holding the
-            // pair (t % 8) ^ (row & 7); row & 7 does not depend on q
-            const int lrow = t >> 3, lpair = (t & 7) ^ (lrow & 7);
-            p = x + (r0 + lrow) * ld + 2 * lpair;
-        } else {
-            p = x + r0 + 2 * lane;
-        }
-    }
-    __device__ __forceinline__ void issue(int64_t k0, double *tile) const {
-        const int wave = threadIdx.x >> 6;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            if (KCONTIG) lds_dma16(p + q * 32 * ld + k0, tile + 2 * (q * 256 + 64 * wave));
-            else lds_dma16(p + (k0 + 4 * q + wave) * ld, tile + (4 * q + wave) * RC_LD);
-        }
-    }
-    __device__ __forceinline__ static f64x2 frag(const double *tile, int r, int kp) {
-        if (KCONTIG) return *reinterpret_cast<const f64x2 *>(tile + 2 * (r * KP + (kp ^ (r & 7))));
-        return f64x2{tile[2 * kp * RC_LD + r], tile[(2 * kp + 1) * RC_LD + r]};
-    }
-};
-
-template <bool AK, bool BKC>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void dgemm_dl_kernel(
-    int64_t M, int64_t N, int64_t K, double alpha,
-    const double *__restrict__ A, int64_t lda,
-    const double *__restrict__ B, int64_t ldb,
-    double beta, double *__restrict__ C, int64_t ldc,
-    int vec_c, int group_m) {
-    using OA = DlOperand<AK>;
-    using OB = DlOperand<BKC>;
-    constexpr int STAGE = OA::SIZE + OB::SIZE;
-    __shared__ __attribute__((aligned(16))) double sm[2][STAGE];   // 64-68 KB
-    constexpr int FM = 4, FN = 4;
-    const int64_t tiles_m = M / DL_TILE, tiles_n = N / DL_TILE;
-    const int64_t bid = xcd_remap(blockIdx.x, tiles_m * tiles_n);
-    const int64_t per_group = (int64_t)group_m * tiles_n;
-    const int64_t grp = bid / per_group;
-    const int64_t first_m = grp * group_m;
-    const int64_t gsize = min((int64_t)group_m, tiles_m - first_m);
-    const int64_t in_group = bid - grp * per_group;
-    const int64_t m0 = (first_m + in_group % gsize) * DL_TILE;
-    const int64_t n0 = (in_group / gsize) * DL_TILE;
-
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
-    const int g = lane >> 4, li = lane & 15;
-    const int abase = wm * 64 + 4 * (li & 3) + (li >> 2);
-    const int bbase = wn * 64 + li;
-    const OA oa(A, lda, m0);
-    const OB ob(B, ldb, n0);
-    const int64_t nk = K / BK;
-    auto issue = [&](int64_t kt, int st) {
-        oa.issue(kt * BK, sm[st]);
-        ob.issue(kt * BK, sm[st] + OA::SIZE);
-    };
-
-    f64x4 acc[FM][FN];
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(0.0, 0.0, f64x4{0.0, 0.0, 0.0, 0.0}, 0, 0, 0);
-    f64x2 af[2][FM], bf[2][FN];
-    auto read_frags = [&](int st, int ks, int h) {
-        const int kp = 4 * ks + g;
-#pragma unroll
-        for (int i = 0; i < FM; ++i) af[h][i] = OA::frag(sm[st], abase + 16 * i, kp);
-#pragma unroll
-        for (int j = 0; j < FN; ++j) bf[h][j] = OB::frag(sm[st] + OA::SIZE, bbase + 16 * j, kp);
-    };
-    // MFMAs [from, to) of sub-step h, in gemm_tile's order: the .x block
-    // (k = 2 kp), then the .y block (k = 2 kp + 1), each row-major in (i, j)
-    auto mfma_range = [&](int h, int from, int to) {
-#pragma unroll
-        for (int q = 0; q < 2 * FM * FN; ++q) {
-            if (q < from || q >= to) continue;
-            const int i = (q % (FM * FN)) / FN, j = q % FN;
-            if (q < FM * FN) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[h][i].x, bf[h][j].x, acc[i][j], 0, 0, 0);
-            else acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[h][i].y, bf[h][j].y, acc[i][j], 0, 0, 0);
-        }
-    };
-    // Entering iteration kt: stage kt & 1 holds step kt and F[0] its first
-    // sub-step; the loads of step kt + 1 into the other stage are in flight.
-    // Iteration: read sub-step 1 into F[1]; MFMAs of F[0]; wait for this
-    // wave's loads (step kt + 1) and barrier (every wave's loads have landed
-    // and every wave has read step kt); refill stage kt & 1 with step kt + 2
-    // (the last steps reload step nk - 1, never read: no branch); read the
-    // first sub-step of step kt + 1 into F[0]; MFMAs of F[1].  The MFMAs of
-    // F[1] after the barrier cover the latency of the F[0] reads, and those
-    // of F[0] before it the latency of the F[1] reads, so the barrier's own
-    // LDS wait finds nothing outstanding.  The scheduling barriers hold that
-    // order: left alone the compiler moved the MFMAs past the barrier and
-    // the fragment reads up to it, so that the barrier waited for the reads
-    // with the MFMA pipe idle.  With both operands k-contiguous (A 'T',
-    // B 'N') the F[1] reads measured fastest issued as one batch ahead of
-    // all F[0] MFMAs (+1.5% against the compiler's order at 8192^3 and
-    // 16384^3), for the other layouts behind the first four F[0] MFMAs
-    // (+0.2-0.5%; the batch form there 0.3% slower).
-    auto iteration = [&](int64_t kt, int st) {
-        constexpr int HEAD = (AK && BKC) ? 0 : 4;
-        mfma_range(0, 0, HEAD);
-        __builtin_amdgcn_sched_barrier(0);
-        read_frags(st, 1, 1);
-        __builtin_amdgcn_sched_barrier(0);
-        mfma_range(0, HEAD, 2 * FM * FN);
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(WAIT_VMCNT0);
-        __syncthreads();
-        issue(min(kt + 2, nk - 1), st);
-        read_frags(st ^ 1, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        mfma_range(1, 0, 2 * FM * FN);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    issue(0, 0);
-    issue(min((int64_t)1, nk - 1), 1);
-    __builtin_amdgcn_s_waitcnt(WAIT_VMCNT0 | 8);   // vmcnt(8): step 0 landed
-    __syncthreads();
-    read_frags(0, 0, 0);
-    int64_t kt = 0;
-    for (; kt + 1 < nk; kt += 2) {
-        iteration(kt, 0);
-        iteration(kt + 1, 1);
-    }
-    if (kt < nk) iteration(kt, 0);
-    __builtin_amdgcn_s_waitcnt(WAIT_VMCNT0);   // no LDS writes outstanding at exit
-
-    // ---- epilogue (gemm_tile's): lane holds rows 4g..4g+3 of column li
-    const bool beta0 = (beta == 0.0);
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-        const int64_t row = m0 + wm * 64 + 16 * i + 4 * g;
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            const int64_t col = n0 + wn * 64 + 16 * j + li;
-            double *cp = C + row + col * ldc;
-            const f64x4 r = acc[i][j];
-            if (vec_c) {
-                f64x2 *cv = reinterpret_cast<f64x2 *>(cp);
-                f64x2 lo = {alpha * r[0], alpha * r[1]};
-                f64x2 hi = {alpha * r[2], alpha * r[3]};
-                if (!beta0) {
-                    const f64x2 clo = cv[0], chi = cv[1];
-                    lo.x = fma(beta, clo.x, lo.x); lo.y = fma(beta, clo.y, lo.y);
-                    hi.x = fma(beta, chi.x, hi.x); hi.y = fma(beta, chi.y, hi.y);
-                }
-                cv[0] = lo;
-                cv[1] = hi;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    double val = alpha * r[e];
-                    if (!beta0) val = fma(beta, cp[e], val);
-                    cp[e] = val;
-                }
-            }
-        }
-    }
-}
-
 // Grouped tiles without LDS ("direct"): one wave per (16 FI) x (16 FJ) C tile
 // (64 x 64 or 32 x 32: up to FI x FJ blocks of 16 x 16 in AGPR accumulators;
 // blocks outside C are skipped),
@@ -904,32 +701,9 @@ int launch_add_scaled(int64_t m, int64_t n, double beta, const double *x, int64_
     return COSMA_AMD_OK;
 }
 
-// The direct-LDS kernel's conditions (see dgemm_dl_kernel).
-bool dl_eligible(int64_t m, int64_t n, int64_t k, const double *a, int64_t lda, const double *b, int64_t ldb) {
-    return m % DL_TILE == 0 && n % DL_TILE == 0 && k % BK == 0 && k > 0 && aligned16(a) && aligned16(b) &&
-           lda % 2 == 0 && ldb % 2 == 0 && (m / DL_TILE) * (n / DL_TILE) <= 0x7fffffffLL;
-}
-
-int launch_dl(char ta, char tb, int64_t m, int64_t n, int64_t k, double alpha, const double *a, int64_t lda,
-              const double *b, int64_t ldb, double beta, double *c, int64_t ldc, int group_m, hipStream_t s) {
-    const int vec_c = aligned16(c) && (ldc % 2 == 0);
-    const dim3 grid((unsigned)((m / DL_TILE) * (n / DL_TILE))), block(NT);
-#define CA_LAUNCH_DL(X, Y)                                                                                 \
-    hipLaunchKernelGGL((dgemm_dl_kernel<X, Y>), grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, \
-                       ldc, vec_c, group_m)
-    // template flags: operand k-contiguous (A 'T', B 'N')
-    if (ta == 'T' && tb == 'N') CA_LAUNCH_DL(true, true);
-    else if (ta == 'N' && tb == 'N') CA_LAUNCH_DL(false, true);
-    else if (ta == 'N' && tb == 'T') CA_LAUNCH_DL(false, false);
-    else CA_LAUNCH_DL(true, false);
-#undef CA_LAUNCH_DL
-    CA_HIP(hipGetLastError());
-    return COSMA_AMD_OK;
-}
-
 // Tile configuration: 0 = automatic, 1 = 128x128, 2 = 256x128, 3 = 128x256,
-// 4 = the direct-LDS kernel (128x128, two workgroups per CU) where its
-// conditions hold, else as 0.
+// 4 = the direct-LDS kernel's 128x128 tile for whole tiles of 16-byte aligned
+// operands, else as 0.
 static int g_cfg_override = 0;
 static int g_group_override = 0;
 
@@ -938,31 +712,19 @@ int launch_dgemm_cfg(int cfg, int group_m, char ta, char tb, int64_t m, int64_t 
                      double beta, double *c, int64_t ldc, hipStream_t s) {
     if (m == 0 || n == 0) return COSMA_AMD_OK;
     if (k == 0 || alpha == 0.0) return launch_scale(m, n, beta, c, ldc, s);
-    // Large tiles need enough of them to fill 256 CUs; of the two large
-    // shapes 128 x 256 measured faster for NN and TN at 8192^3 and 16384^3.
-    const int64_t t_large = ((m + 127) / 128) * ((n + 255) / 256);
-    const int auto_cfg = (t_large >= 512) ? 3 : 1;
-    if (cfg == 4 || cfg == 0) {
-        // The direct-LDS kernel (bit-identical results) against 128 x 256
-        // tiles at 8192^3 / 16384^3 measured +5% / +4% (NN), +3% / +2.7%
-        // (TN), +6% / +6% (NT), +3% / +3% (TT).  With 512 tiles resident (two
-        // per CU) against 256, its last, partial round can waste more: it is
-        // taken automatically from 1024 tiles on, unless the other choice's
-        // last round is fuller by more than its 4% advantage.
-        bool take = cfg == 4;
-        if (!take && dl_eligible(m, n, k, a, lda, b, ldb)) {
-            const int64_t t = (m / DL_TILE) * (n / DL_TILE);
-            const int64_t t_alt = auto_cfg == 3 ? t_large : ((m + 127) / 128) * ((n + 127) / 128);
-            auto fill = [](int64_t tiles, int64_t slots) {
-                return (double)tiles / (double)(((tiles + slots - 1) / slots) * slots);
-            };
-            take = t >= 1024 && 1.04 * fill(t, 512) >= fill(t_alt, 256);
-        }
-        if (take && dl_eligible(m, n, k, a, lda, b, ldb))
-            return launch_dl(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, group_m > 0 ? group_m : 8, s);
+    if (cfg == 4 && !(m % 128 == 0 && n % 128 == 0 && k % BK == 0 && aligned16(a) && aligned16(b) && lda % 2 == 0 &&
+                      ldb % 2 == 0))
         cfg = 0;
+    if (cfg == 4 || cfg == 0) {
+        // The direct-LDS kernel against this file's tiles: 8192^3 NN 72.1 vs
+        // 67.5 TF, 2000^3 NN 245 vs 266 us, 100^3 4.4 vs 19.7 us; those remain
+        // for what its 32-bit offsets cannot reach.
+        if (dl_fits(m, n, k, lda, ldb)) {
+            const DlTile tile = cfg == 4 ? DL_128x128 : pick_dl_tile(m, n, k);
+            return launch_dl(tile, ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, group_m > 0 ? group_m : 8, s);
+        }
+        cfg = ((m + 127) / 128) * ((n + 255) / 256) >= 512 ? 3 : 1;
     }
-    if (cfg == 0) cfg = auto_cfg;
     switch (cfg) {
     case 1: return launch_cfg<128, 128>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, group_m > 0 ? group_m : 8, s);
     case 2: return launch_cfg<256, 128>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, group_m > 0 ? group_m : 4, s);

@@ -1,0 +1,389 @@
+// FP64 DGEMM on the gfx950 matrix cores with operand tiles loaded straight
+// from global memory into LDS (global_load_lds_dwordx4: lane l of a wave
+// instruction writes the 16 bytes at the instruction's LDS base + 16 l), for
+// any extents, leading dimensions and transposes.  The default kernel of
+// cosma_amd_dgemm.
+//
+//   * A workgroup of 2 x 2 waves owns a BM x BN tile of C, a wave a quarter of
+//     it in 16 x 16 MFMA blocks.  Five tile shapes, 128 x 128 to 32 x 32, all
+//     summing k in the order of dgemm.hip's gemm_tile: the choice of a tile
+//     (pick_dl_tile) never changes a bit of the result.
+//   * What bounds it: the FP64 MFMA pipe (a v_mfma_f64_16x16x4 takes 64
+//     cycles of a SIMD).  Two to four workgroups per CU share the pipe, so one's
+//     barrier and fragment reads overlap the others' MFMAs; NS LDS stages keep
+//     the loads of the next NS - 1 steps in flight, which is what a CU with a
+//     single workgroup needs (1024 x 1024 x 32768 TN, one 64 x 64 tile per CU:
+//     1332 us with two stages, 1000 us with three).
+//   * Fragment registers are double-buffered by half-step, and each batch of
+//     reads is waited for before the next one is issued (by then 8 to 32
+//     MFMAs old).  Left to the compiler, the wait stood behind the next batch
+//     and covered it too, idling the wave for an LDS round trip per half-step
+//     (8192^3 TN 70.6 -> 73.0 TF, NN 70.7 -> 72.1 with the scalar addresses).
+//   * LDS layout per operand and stage, both free of bank conflicts:
+//     k-contiguous (A 'T', B 'N'): row r holds its eight k-pairs in 128 bytes,
+//     pair kp in slot kp ^ row_swz(r); a fragment is one 16-byte read.
+//     Row-contiguous (A 'N', B 'T'): k-row k holds the tile's rows, row r at
+//     r ^ (16 if its k-pair is odd); a fragment is two 8-byte reads.
+//     The loads' global addresses apply the permutations.
+//   * Edges: rows beyond the matrix are read from its last row (or row pair)
+//     and their results never stored, so full steps need no masks; the
+//     partial last step is loaded by element, zero beyond K.  16-byte accesses
+//     need no more than the 8-byte alignment of a double.
+#include <algorithm>
+
+#include "common.hpp"
+#include "dgemm_dl.hpp"
+
+namespace cosma_amd {
+namespace {
+
+constexpr int BK = 16;       // k-step
+constexpr int NT = 256;      // threads per workgroup: 2 x 2 waves
+constexpr int NXCD = 8;
+
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));   // 16-byte access at 8-byte alignment
+
+// s_waitcnt immediates (gfx9 fields: vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
+constexpr int wait_vm(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0F70; }
+constexpr int WAIT_LGKM0 = 0xC07F;
+constexpr int WAIT_VM0_LGKM0 = 0x0070;
+
+// Slot (of eight) of k-pair kp in row r of a k-contiguous tile is kp ^ row_swz(r).
+__device__ __forceinline__ int row_swz(int r) { return ((r >> 2) & 3) | ((r & 2) << 1); }
+
+template <int R, bool KCONTIG>
+struct Operand {
+    static constexpr int SIZE = R * BK;          // doubles per stage
+    static constexpr int LOADS = R / 32;         // 1 KB wave instructions per wave and step
+    static constexpr int NOFF = KCONTIG ? LOADS : 1;
+    static constexpr int TAIL = R * BK / NT;     // elements per thread of the partial step
+    const char *base;                            // wave-uniform
+    int64_t ldb;                                 // leading dimension in bytes
+    uint32_t off[NOFF];                          // per-lane byte offsets
+
+    __device__ __forceinline__ Operand(const double *x, int64_t ld, int64_t r0, int64_t ext, int wave, int lane) {
+        ldb = ld * 8;
+        const int last = (int)min((int64_t)(R - 1), ext - 1 - r0);   // last row of the tile inside the matrix
+        if (KCONTIG) {
+            base = reinterpret_cast<const char *>(x + r0 * ld);
+#pragma unroll
+            for (int q = 0; q < LOADS; ++q) {
+                const int row = 8 * (wave + 4 * q) + (lane >> 3);
+                off[q] = (uint32_t)min(row, last) * (uint32_t)ldb + (uint32_t)(((lane & 7) ^ row_swz(row)) * 16);
+            }
+        } else {
+            const int e = 2 * lane;                                  // position in the 128 doubles of an instruction
+            const int kl = e / R, pos = e % R;
+            const int odd_kp = R == 128 ? (wave >> 1) & 1 : R == 64 ? wave & 1 : lane >> 5;
+            const int row = min(pos ^ (16 * odd_kp), last & ~1);
+            base = reinterpret_cast<const char *>(x + r0) + (int64_t)(wave * (128 / R)) * ldb;
+            off[0] = (uint32_t)kl * (uint32_t)ldb + (uint32_t)row * 8;
+        }
+    }
+    __device__ __forceinline__ void issue(int k0, double *tile, int wave) const {
+#pragma unroll
+        for (int q = 0; q < LOADS; ++q) {
+            // scalar base + 32-bit lane offset (the asm keeps the compiler from
+            // folding the lane offset into 64-bit vector adds per load)
+            const char *u = KCONTIG ? base + (int64_t)k0 * 8 : base + (int64_t)(k0 + q * (512 / R)) * ldb;
+            asm("" : "+s"(u));
+            __builtin_amdgcn_global_load_lds(static_cast<const void *>(u + off[KCONTIG ? q : 0]),
+                                             (__attribute__((address_space(3))) void *)(tile + 128 * (wave + 4 * q)),
+                                             16, 0, 0);
+        }
+    }
+    // The partial step: elements (row, k) with k < kt, zero beyond.
+    __device__ __forceinline__ static void tail_rk(int e, int &row, int &k) {
+        const int idx = threadIdx.x + NT * e;
+        if (KCONTIG) { row = idx >> 4; k = idx & 15; }
+        else { row = idx % R; k = idx / R; }
+    }
+    __device__ __forceinline__ static void tail_load(const double *x, int64_t ld, int64_t r0, int64_t ext, int64_t k0,
+                                                     int kt, double (&v)[TAIL]) {
+        const int last = (int)min((int64_t)(R - 1), ext - 1 - r0);
+#pragma unroll
+        for (int e = 0; e < TAIL; ++e) {
+            int row, k;
+            tail_rk(e, row, k);
+            const int64_t r = r0 + min(row, last);
+            v[e] = k < kt ? (KCONTIG ? x[k0 + k + r * ld] : x[r + (k0 + k) * ld]) : 0.0;
+        }
+    }
+    __device__ __forceinline__ static void tail_store(double *tile, const double (&v)[TAIL]) {
+#pragma unroll
+        for (int e = 0; e < TAIL; ++e) {
+            int row, k;
+            tail_rk(e, row, k);
+            tile[KCONTIG ? 2 * (row * 8 + ((k >> 1) ^ row_swz(row))) + (k & 1) : k * R + (row ^ (16 * ((k >> 1) & 1)))] =
+                v[e];
+        }
+    }
+};
+
+// Fragment reads of one operand: row base + 16 i, lane group g, sub-step ks
+// (k-pair kp = 4 ks + g).
+template <int R, bool KCONTIG>
+struct Frag {
+    int o0, o1;
+    __device__ __forceinline__ Frag(int rbase, int g) {
+        if (KCONTIG) {
+            o0 = 2 * (rbase * 8 + (g ^ row_swz(rbase)));
+            o1 = 2 * (rbase * 8 + ((g + 4) ^ row_swz(rbase)));
+        } else {
+            const int gb = 16 * (g & 1);
+            o0 = 2 * g * R + (R == 32 ? rbase ^ gb : rbase + gb);   // even i
+            o1 = 2 * g * R + rbase - gb;                            // odd i
+        }
+    }
+    __device__ __forceinline__ f64x2 read(const double *tile, int i, int ks) const {
+        if (KCONTIG) return *reinterpret_cast<const f64x2 *>(tile + (ks ? o1 : o0) + 256 * i);
+        const double *p = tile + ((i & 1) ? o1 : o0) + 16 * i + 8 * ks * R;
+        return f64x2{p[0], p[R]};
+    }
+};
+
+// NS: LDS stages; WPE: waves per SIMD (= workgroups per CU) it is built for.
+template <int BM, int BN, int NS, int WPE, bool AK, bool BKC>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void dgemm_dl_kernel(
+    int64_t M, int64_t N, int64_t K, double alpha,
+    const double *__restrict__ A, int64_t lda,
+    const double *__restrict__ B, int64_t ldb,
+    double beta, double *__restrict__ C, int64_t ldc, int group_m) {
+    using OA = Operand<BM, AK>;
+    using OB = Operand<BN, BKC>;
+    constexpr int STAGE = OA::SIZE + OB::SIZE;
+    constexpr int LOADS = OA::LOADS + OB::LOADS;
+    constexpr int FM = BM / 32, FN = BN / 32;
+    constexpr bool EARLY_TAIL = BM * BN <= 64 * 64;
+    __shared__ __attribute__((aligned(16))) double sm[NS * STAGE];
+
+    // ---- tile rasterisation (XCD-aware, grouped along m)
+    const uint32_t tiles_m = (uint32_t)((M + BM - 1) / BM), tiles_n = (uint32_t)((N + BN - 1) / BN);
+    const uint32_t T = gridDim.x, q8 = T / NXCD, r8 = T % NXCD, xcd = blockIdx.x % NXCD, loc = blockIdx.x / NXCD;
+    const uint32_t bid = xcd * q8 + min(xcd, r8) + loc;
+    const uint32_t per_group = group_m * tiles_n, grp = bid / per_group, in_group = bid - grp * per_group;
+    const uint32_t gsize = min((uint32_t)group_m, tiles_m - grp * group_m);
+    const int64_t m0 = (int64_t)(grp * group_m + in_group % gsize) * BM;
+    const int64_t n0 = (int64_t)(in_group / gsize) * BN;
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    const int g = lane >> 4, li = lane & 15;
+    const OA oa(A, lda, m0, M, wave, lane);
+    const OB ob(B, ldb, n0, N, wave, lane);
+    const Frag<BM, AK> fra(wm * (BM / 2) + 4 * (li & 3) + (li >> 2), g);
+    const Frag<BN, BKC> frb(wn * (BN / 2) + li, g);
+
+    // Full steps; a row-contiguous operand with an odd extent keeps the last
+    // k out of them (the 16-byte load of its last row reads one element
+    // beyond the row, which only inside the matrix is the next column's).
+    const bool hold_last = (!AK && (M & 1)) || (!BKC && (N & 1));
+    const int nk = (int)((hold_last ? K - 1 : K) / BK);
+    const int kt = (int)(K - (int64_t)nk * BK);   // 0..16
+    double ta[OA::TAIL], tb[OB::TAIL];
+    auto tail_load = [&]() {
+        OA::tail_load(A, lda, m0, M, (int64_t)nk * BK, kt, ta);
+        OB::tail_load(B, ldb, n0, N, (int64_t)nk * BK, kt, tb);
+    };
+
+    f64x4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+    f64x2 af[2][FM], bf[2][FN];
+    auto read_frags = [&](const double *tile, int ks) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i) af[ks][i] = fra.read(tile, i, ks);
+#pragma unroll
+        for (int j = 0; j < FN; ++j) bf[ks][j] = frb.read(tile + OA::SIZE, j, ks);
+    };
+    auto mfmas = [&](int h) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[h][i].x, bf[h][j].x, acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[h][i].y, bf[h][j].y, acc[i][j], 0, 0, 0);
+    };
+    auto issue = [&](int kt_, double *tile) {
+        oa.issue(kt_ * BK, tile, wave);
+        ob.issue(kt_ * BK, tile + OA::SIZE, wave);
+    };
+    auto barrier = [&]() {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    if (EARLY_TAIL && kt > 0) tail_load();
+
+    if (nk > 0) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) issue(min(s, nk - 1), sm + s * STAGE);
+        __builtin_amdgcn_s_waitcnt(wait_vm((NS - 1) * LOADS));
+        barrier();
+        read_frags(sm, 0);
+        auto iteration = [&](int k, double *cur, double *next) {
+            __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);
+            __builtin_amdgcn_sched_barrier(0);
+            read_frags(cur, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            mfmas(0);
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(wait_vm((NS - 2) * LOADS) & WAIT_LGKM0);
+            barrier();
+            issue(min(k + NS, nk - 1), cur);
+            __builtin_amdgcn_sched_barrier(0);
+            read_frags(next, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            mfmas(1);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        int k = 0;
+        for (; k + NS <= nk; k += NS) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) iteration(k + s, sm + s * STAGE, sm + ((s + 1) % NS) * STAGE);
+        }
+#pragma unroll
+        for (int s = 0; s < NS - 1; ++s)
+            if (k + s < nk) iteration(k + s, sm + s * STAGE, sm + ((s + 1) % NS) * STAGE);
+    }
+    if (kt > 0) {
+        if (!EARLY_TAIL) tail_load();
+        __builtin_amdgcn_s_waitcnt(WAIT_VM0_LGKM0);   // no load into LDS outstanding
+        barrier();
+        OA::tail_store(sm, ta);
+        OB::tail_store(sm + OA::SIZE, tb);
+        __syncthreads();
+        read_frags(sm, 0);
+        read_frags(sm, 1);
+        mfmas(0);
+        mfmas(1);
+    }
+    __builtin_amdgcn_s_waitcnt(wait_vm(0));   // no LDS writes outstanding at exit
+
+    // ---- epilogue: lane holds rows 4g..4g+3 (contiguous) of column li
+    const bool beta0 = (beta == 0.0);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+        const int64_t row = m0 + wm * (BM / 2) + 16 * i + 4 * g;
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            const int64_t col = n0 + wn * (BN / 2) + 16 * j + li;
+            if (col >= N) continue;
+            double *cp = C + row + col * ldc;
+            const f64x4 r = acc[i][j];
+            if (row + 3 < M) {
+                f64x2u *cv = reinterpret_cast<f64x2u *>(cp);
+                f64x2u lo = {alpha * r[0], alpha * r[1]};
+                f64x2u hi = {alpha * r[2], alpha * r[3]};
+                if (!beta0) {
+                    const f64x2u clo = cv[0], chi = cv[1];
+                    lo.x = fma(beta, clo.x, lo.x); lo.y = fma(beta, clo.y, lo.y);
+                    hi.x = fma(beta, chi.x, hi.x); hi.y = fma(beta, chi.y, hi.y);
+                }
+                cv[0] = lo;
+                cv[1] = hi;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (row + e < M) {
+                        double val = alpha * r[e];
+                        if (!beta0) val = fma(beta, cp[e], val);
+                        cp[e] = val;
+                    }
+                }
+            }
+        }
+    }
+}
+
+template <int BM, int BN, int NS, int WPE>
+void launch(char ta, char tb, int64_t m, int64_t n, int64_t k, double alpha, const double *a, int64_t lda,
+            const double *b, int64_t ldb, double beta, double *c, int64_t ldc, int group_m, hipStream_t s) {
+    const dim3 grid((unsigned)(((m + BM - 1) / BM) * ((n + BN - 1) / BN))), block(NT);
+#define CA_LAUNCH_DL(X, Y)                                                                                        \
+    hipLaunchKernelGGL((dgemm_dl_kernel<BM, BN, NS, WPE, X, Y>), grid, block, 0, s, m, n, k, alpha, a, lda, b,   \
+                       ldb, beta, c, ldc, group_m)
+    // template flags: operand k-contiguous (A 'T', B 'N')
+    if (ta == 'T' && tb == 'N') CA_LAUNCH_DL(true, true);
+    else if (ta == 'N' && tb == 'N') CA_LAUNCH_DL(false, true);
+    else if (ta == 'N' && tb == 'T') CA_LAUNCH_DL(false, false);
+    else CA_LAUNCH_DL(true, false);
+#undef CA_LAUNCH_DL
+}
+
+}  // namespace
+
+namespace {
+constexpr int N_CU = 256;
+struct TileModel {
+    int bm, bn;
+    double extra;     // prologue and epilogue of a tile, in k
+    double busy[3];   // MFMA utilisation with one, two, and more tiles per CU
+};
+// Fitted to 410 shapes (m, n 32 to 8192, k 8 to 32768, all transposes and
+// alignments, every tile timed): the choice is 0.6% slower than the fastest
+// tile on average, 14% at most.
+constexpr TileModel MODEL[] = {
+    {128, 128, 210, {0.91, 0.913, 0.92}}, {64, 128, 98, {0.55, 0.66, 0.886}}, {64, 64, 62, {0.75, 0.785, 0.877}},
+    {64, 32, 60, {0.65, 0.70, 0.789}},    {32, 32, 56, {0.59, 0.654, 0.689}},
+};
+int64_t tiles_of(DlTile t, int64_t m, int64_t n) {
+    return ((m + MODEL[t].bm - 1) / MODEL[t].bm) * ((n + MODEL[t].bn - 1) / MODEL[t].bn);
+}
+}  // namespace
+
+// The busiest CU computes ceil(tiles / CUs) tiles, each bm * bn * (k + extra)
+// products at the tile's MFMA utilisation: large tiles move less data per
+// product, small ones leave less of the chip idle and pad less.  1000^3 NN:
+// 132 us in 128 x 128 tiles (64 of 256 CUs busy), 38 us in 64 x 64; 1537 x
+// 1021 x 2999 NT: 381 us, 171 us in 32 x 32; 8192^3 NN: 15.2 ms, 18.6 ms.
+DlTile pick_dl_tile(int64_t m, int64_t n, int64_t k) {
+    DlTile best = DL_128x128;
+    double least = 0.0;
+    for (int t = DL_128x128; t <= DL_32x32; ++t) {
+        const TileModel &x = MODEL[t];
+        const int64_t per_cu = (tiles_of(static_cast<DlTile>(t), m, n) + N_CU - 1) / N_CU;
+        const double cost = (double)(per_cu * x.bm * x.bn) * ((double)k + x.extra) / x.busy[std::min<int64_t>(per_cu, 3) - 1];
+        if (t == DL_128x128 || cost < least) {
+            least = cost;
+            best = static_cast<DlTile>(t);
+        }
+    }
+    return best;
+}
+
+bool dl_fits(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb) {
+    // 32-bit byte offsets over 128 rows, 32-bit step counts, and the 2^32
+    // work-items of a launch in the smallest tiles
+    return (m + 31) / 32 * ((n + 31) / 32) < ((int64_t)1 << 24) && k < ((int64_t)1 << 31) &&
+           lda < ((int64_t)1 << 22) && ldb < ((int64_t)1 << 22);
+}
+
+int launch_dl(DlTile tile, char ta, char tb, int64_t m, int64_t n, int64_t k, double alpha, const double *a, int64_t lda,
+              const double *b, int64_t ldb, double beta, double *c, int64_t ldc, int group_m, hipStream_t s) {
+#define CA_DL(BM, BN, NS, WPE) \
+    launch<BM, BN, NS, WPE>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, group_m, s)
+    switch (tile) {
+    case DL_128x128: CA_DL(128, 128, 2, 2); break;
+    case DL_64x128: CA_DL(64, 128, 2, 3); break;
+    case DL_64x64: {
+        // one tile per CU and fewer: a third stage in place of the other workgroups
+        if (tiles_of(DL_64x64, m, n) <= N_CU) CA_DL(64, 64, 3, 3);
+        else CA_DL(64, 64, 2, 4);
+        break;
+    }
+    case DL_64x32: CA_DL(64, 32, 3, 4); break;
+    default: CA_DL(32, 32, 4, 4); break;
+    }
+#undef CA_DL
+    CA_HIP(hipGetLastError());
+    return COSMA_AMD_OK;
+}
+
+}  // namespace cosma_amd
