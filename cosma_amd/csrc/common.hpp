@@ -194,4 +194,12 @@ int launch_fill_lognormal(double *x, int64_t rows, int64_t cols, int64_t ld, uin
 int launch_block_transform(char op, int64_t rows, int64_t cols, double alpha,
                            const double *src, int64_t lds, double beta,
                            double *dst, int64_t ldd, hipStream_t s);
+// dst <- alpha * src + beta * dst for many device blocks (column-major, no
+// two dst blocks overlapping).
+struct CopyBlock {
+    const double *src;
+    double *dst;
+    int64_t lds, ldd, rows, cols;
+};
+int launch_block_copies(const CopyBlock *blocks, int64_t n, double alpha, double beta, hipStream_t s);
 }  // namespace cosma_amd

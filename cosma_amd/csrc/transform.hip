@@ -9,17 +9,27 @@
 // (numroc with one process returns the full extent, src/cosma/scalapack.cpp:49-87),
 // so the reorder reduces to this strided copy / transpose.
 //
-// op = 'N': each thread streams 2 consecutive doubles of a column (16-byte
-//           accesses when both leading dimensions and pointers allow it).
-// op = 'T': 64 x 64 tiles staged through LDS with a one-double row pad, so
-//           both the read of src and the write of dst walk memory contiguously
-//           (rows of the tile are read along src columns and written along
-//           dst columns); the pad spreads the column reads over all banks.
-//           With aligned pointers and even leading dimensions the global
-//           accesses are 16 bytes wide (two consecutive elements) and
-//           non-temporal (4.87 -> 5.2 TB/s in the probe of the variants), and
-//           a workgroup takes several tiles of a column, loading the next
-//           one while it writes the current one (16384^2: 0.865 -> 0.835 ms).
+// The bound is HBM.  With a leading dimension that is no multiple of 16 the
+// columns of dst start anywhere in a 128-byte line, and the lines at the ends
+// of a tile's column runs are written in parts by two workgroups.  So the
+// copies and the large transposes give every column of dst its own row
+// window, which starts where a line does, and use 16-byte accesses at the
+// 8-byte alignment of a double (8191 x 12289, ld 12291 / 8193: 'T' 421 us
+// element by element, 358 us in 16-byte accesses, 298 us in shifted windows =
+// 5.4 TB/s; 'N' 351 -> 250 us = 6.4 TB/s).
+//
+// op = 'N': a workgroup covers 512 rows of one or two columns, a thread two
+//           consecutive doubles of each.
+// op = 'T': tiles staged through LDS (odd row pitch, so that the column reads
+//           spread over all banks): read along src columns, written along dst
+//           columns.  Three forms: operands that the last-level cache holds in
+//           64 x 64 tiles (with aligned pointers and even leading dimensions
+//           16-byte accesses, and several tiles per workgroup, the next loaded
+//           during the stores of the current one); larger ones in shifted
+//           windows, which need 16 more src columns than they write rows (the
+//           next tile's too, from L2: their loads are cached); and larger ones
+//           with all columns in whole lines in 128 x 64 tiles that stream past
+//           the caches on both sides.
 // alpha == 1 and beta == 0 copies values bit-for-bit (no arithmetic at all);
 // beta == 0 never reads dst.
 #include "common.hpp"
@@ -27,8 +37,10 @@
 namespace cosma_amd {
 namespace {
 
-constexpr int TT = 64;       // transpose tile edge
-constexpr int TNT = 256;     // threads per transpose workgroup
+constexpr int LINE = 16;     // doubles per 128-byte line
+constexpr int NT = 256;      // threads per workgroup
+
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
 
 __device__ __forceinline__ double combine(double x, double alpha, double beta, const double *d, int mode) {
     // mode 0: pure copy; 1: alpha*x (dst not read); 2: alpha*x + beta*dst
@@ -36,48 +48,119 @@ __device__ __forceinline__ double combine(double x, double alpha, double beta, c
     if (mode == 1) return alpha * x;
     return fma(beta, *d, alpha * x);
 }
+__device__ __forceinline__ f64x2u combine2(f64x2u x, double alpha, double beta, f64x2u old, int mode) {
+    if (mode == 0) return x;
+    if (mode == 1) return f64x2u{alpha * x.x, alpha * x.y};
+    return f64x2u{fma(beta, old.x, alpha * x.x), fma(beta, old.y, alpha * x.y)};
+}
+// Position of an element in its 128-byte line.
+__device__ __forceinline__ int phase(const double *p) { return (int)(reinterpret_cast<uintptr_t>(p) >> 3) & (LINE - 1); }
 
-// dst(rows x cols) <- f(src(rows x cols)).  Grid: x over row-pairs, y over
-// pairs of columns: a thread loads its two 16-byte pieces (one per column)
-// before it stores either, and the streamed data bypass the caches
-// (non-temporal loads and stores): 16384^2 copy 6.13 -> 6.33 TB/s in a probe
-// of the variants (one column per thread, 2, 4 or 8 columns, flat 1-D).
-__global__ void copy_kernel(int64_t rows, int64_t cols, double alpha,
-                            const double *__restrict__ src, int64_t lds, double beta,
-                            double *__restrict__ dst, int64_t ldd, int mode, int vec) {
-    const int64_t r = 2 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-    if (r >= rows) return;
-    for (int64_t c0 = 2 * (int64_t)blockIdx.y; c0 < cols; c0 += 2 * (int64_t)gridDim.y) {
-        const int nc = c0 + 1 < cols ? 2 : 1;
-        if (vec && r + 1 < rows) {
-            f64x2 v[2];
+// dst(rows x cols) <- f(src(rows x cols)).  Grid: x over 512-row windows, y
+// over columns or pairs of columns.  SHIFT: row windows by dst's lines.
+// STREAM, for operands beyond the last-level cache: one 16-byte piece per
+// thread, all accesses non-temporal (16384^2, beta = 1/2: 1052 -> 992 us;
+// with two pieces 1002 us).  Otherwise two pieces, loaded before either is
+// stored, and cached loads (3000 x 5000: 41 -> 36 us).
+template <bool SHIFT, bool STREAM>
+__global__ __launch_bounds__(NT) void copy_kernel(int64_t rows, int64_t cols, double alpha,
+                                                  const double *__restrict__ src, int64_t lds, double beta,
+                                                  double *__restrict__ dst, int64_t ldd, int mode) {
+    constexpr int U = STREAM ? 1 : 2;
+    auto load2 = [](const double *p) {
+        const f64x2u *q = reinterpret_cast<const f64x2u *>(p);
+        return STREAM ? __builtin_nontemporal_load(q) : *q;
+    };
+    const int64_t r0 = 2 * ((int64_t)blockIdx.x * NT + threadIdx.x);
+    for (int64_t c0 = U * (int64_t)blockIdx.y; c0 < cols; c0 += U * (int64_t)gridDim.y) {
+        f64x2u v[U], old[U];
+        int64_t r[U];
+        bool in[U];
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
-                if (u < nc) v[u] = __builtin_nontemporal_load(reinterpret_cast<const f64x2 *>(src + r + (c0 + u) * lds));
+        for (int u = 0; u < U; ++u) {
+            const int64_t c = c0 + u;
+            r[u] = r0 - (SHIFT ? phase(dst + c * ldd) : 0);
+            in[u] = c < cols && r[u] >= 0 && r[u] + 1 < rows;
+            if (!in[u]) continue;
+            v[u] = load2(src + r[u] + c * lds);
+            if (mode == 2) old[u] = load2(dst + r[u] + c * ldd);
+        }
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                if (u >= nc) continue;
-                double *d = dst + r + (c0 + u) * ldd;
-                f64x2 o;
-                o.x = combine(v[u].x, alpha, beta, d, mode);
-                o.y = combine(v[u].y, alpha, beta, d + 1, mode);
-                __builtin_nontemporal_store(o, reinterpret_cast<f64x2 *>(d));
-            }
-        } else {
-            for (int u = 0; u < nc; ++u) {
-                const double *s = src + r + (c0 + u) * lds;
-                double *d = dst + r + (c0 + u) * ldd;
-                d[0] = combine(s[0], alpha, beta, d, mode);
-                if (r + 1 < rows) d[1] = combine(s[1], alpha, beta, d + 1, mode);
+        for (int u = 0; u < U; ++u) {
+            const int64_t c = c0 + u;
+            double *d = dst + r[u] + c * ldd;
+            if (in[u]) {
+                __builtin_nontemporal_store(combine2(v[u], alpha, beta, old[u], mode), reinterpret_cast<f64x2u *>(d));
+            } else if (c < cols) {
+                const double *q = src + r[u] + c * lds;
+                if (r[u] >= 0 && r[u] < rows) d[0] = combine(q[0], alpha, beta, d, mode);
+                if (r[u] + 1 >= 0 && r[u] + 1 < rows) d[1] = combine(q[1], alpha, beta, d + 1, mode);
             }
         }
     }
 }
 
+// The same for many blocks in one launch: a workgroup takes 2048 consecutive
+// pairs of one block (row pairs of its columns, columns one after another).
+// The block list travels in the kernel arguments: nothing to allocate, upload
+// or keep alive.
+constexpr int LIST = 72;     // blocks per launch (3.5 KB of the 4 KB of arguments)
+constexpr int ITEMS = 8;     // pairs per thread
+struct BlockList {
+    struct {
+        const double *src;
+        double *dst;
+        int64_t lds, ldd;
+        int rows, cols;
+        uint32_t first;      // first workgroup
+        uint32_t pairs;      // row pairs per column, with the window's shift
+    } b[LIST];
+    int n;
+};
+__global__ __launch_bounds__(NT) void copy_list_kernel(BlockList list, double alpha, double beta, int mode) {
+    int lo = 0, hi = list.n - 1;   // last block with first <= this workgroup
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (list.b[mid].first <= blockIdx.x) lo = mid;
+        else hi = mid - 1;
+    }
+    const double *__restrict__ src = list.b[lo].src;
+    double *__restrict__ dst = list.b[lo].dst;
+    const int64_t lds = list.b[lo].lds, ldd = list.b[lo].ldd;
+    const int rows = list.b[lo].rows, cols = list.b[lo].cols;
+    const uint32_t pairs = list.b[lo].pairs, base = (blockIdx.x - list.b[lo].first) * (NT * ITEMS) + threadIdx.x;
+    f64x2u v[ITEMS], old[ITEMS];
+    int r[ITEMS], c[ITEMS];
+    bool in[ITEMS];
+#pragma unroll
+    for (int q = 0; q < ITEMS; ++q) {
+        const uint32_t idx = base + NT * q;
+        c[q] = (int)min(idx / pairs, (uint32_t)cols);
+        r[q] = (int)(2 * (idx - (uint32_t)c[q] * pairs)) - phase(dst + c[q] * ldd);
+        in[q] = c[q] < cols && r[q] >= 0 && r[q] + 1 < rows;
+        if (!in[q]) continue;
+        v[q] = *reinterpret_cast<const f64x2u *>(src + r[q] + c[q] * lds);
+        if (mode == 2) old[q] = *reinterpret_cast<const f64x2u *>(dst + r[q] + c[q] * ldd);
+    }
+#pragma unroll
+    for (int q = 0; q < ITEMS; ++q) {
+        double *d = dst + r[q] + c[q] * ldd;
+        if (in[q]) {
+            __builtin_nontemporal_store(combine2(v[q], alpha, beta, old[q], mode), reinterpret_cast<f64x2u *>(d));
+        } else if (c[q] < cols) {
+            const double *s = src + r[q] + c[q] * lds;
+            if (r[q] >= 0 && r[q] < rows) d[0] = combine(s[0], alpha, beta, d, mode);
+            if (r[q] + 1 >= 0 && r[q] + 1 < rows) d[1] = combine(s[1], alpha, beta, d + 1, mode);
+        }
+    }
+}
+
+constexpr int TT = 64;       // edge of the cached kernels' tiles
+
 // dst(rows x cols)[i, j] <- f(src[j, i]); src is cols x rows with leading dim lds.
 // blockIdx.x -> 64-row block of dst (= 64-column block of src),
 // blockIdx.y -> 64-column block of dst (= 64-row block of src).
-__global__ __launch_bounds__(TNT) void transpose_kernel(int64_t rows, int64_t cols, double alpha,
+__global__ __launch_bounds__(NT) void transpose_cached_kernel(int64_t rows, int64_t cols, double alpha,
                                                         const double *__restrict__ src, int64_t lds,
                                                         double beta, double *__restrict__ dst,
                                                         int64_t ldd, int mode) {
@@ -112,7 +195,7 @@ __global__ __launch_bounds__(TNT) void transpose_kernel(int64_t rows, int64_t co
 // consecutive dst elements of one dst column.  Needs 16-byte aligned
 // pointers and even leading dimensions; tiles that cross the matrix edge take
 // the element-wise path.
-__global__ __launch_bounds__(TNT) void transpose_vec_kernel(int64_t rows, int64_t cols, double alpha,
+__global__ __launch_bounds__(NT) void transpose_cached_vec_kernel(int64_t rows, int64_t cols, double alpha,
                                                             const double *__restrict__ src, int64_t lds,
                                                             double beta, double *__restrict__ dst,
                                                             int64_t ldd, int mode) {
@@ -125,7 +208,7 @@ __global__ __launch_bounds__(TNT) void transpose_vec_kernel(int64_t rows, int64_
     auto load = [&](int64_t j0, f64x2 (&v)[8]) {
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            const int idx = t + TNT * q, il = idx >> 5, c2 = (idx & 31) * 2;
+            const int idx = t + NT * q, il = idx >> 5, c2 = (idx & 31) * 2;
             v[q] = __builtin_nontemporal_load(reinterpret_cast<const f64x2 *>(src + (j0 + c2) + (i0 + il) * lds));
         }
     };
@@ -139,7 +222,7 @@ __global__ __launch_bounds__(TNT) void transpose_vec_kernel(int64_t rows, int64_
         if (full(j0)) {
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                const int idx = t + TNT * q, il = idx >> 5, c2 = (idx & 31) * 2;
+                const int idx = t + NT * q, il = idx >> 5, c2 = (idx & 31) * 2;
                 tile[il][c2] = v[q].x;
                 tile[il][c2 + 1] = v[q].y;
             }
@@ -147,7 +230,7 @@ __global__ __launch_bounds__(TNT) void transpose_vec_kernel(int64_t rows, int64_
             if (j0 + jstep < cols && full(j0 + jstep)) load(j0 + jstep, v);
 #pragma unroll
             for (int q = 0; q < 8; ++q) {     // dst column j0 + jl, rows i0 + r2, r2 + 1
-                const int idx = t + TNT * q, jl = idx >> 5, r2 = (idx & 31) * 2;
+                const int idx = t + NT * q, jl = idx >> 5, r2 = (idx & 31) * 2;
                 f64x2 *d = reinterpret_cast<f64x2 *>(dst + (i0 + r2) + (j0 + jl) * ldd);
                 f64x2 o;
                 if (mode == 0) {
@@ -187,7 +270,77 @@ __global__ __launch_bounds__(TNT) void transpose_vec_kernel(int64_t rows, int64_
     }
 }
 
+// dst(rows x cols)[i, j] <- f(src[j, i]); src is cols x rows with leading dim
+// lds.  Tiles of TR dst rows x TC dst columns, SHIFT: each column's rows start
+// at its own line boundary at or up to 15 rows after the tile's first.
+template <int TR, int TC, bool SHIFT>
+__global__ __launch_bounds__(NT) void transpose_kernel(int64_t rows, int64_t cols, double alpha,
+                                                       const double *__restrict__ src, int64_t lds,
+                                                       double beta, double *__restrict__ dst,
+                                                       int64_t ldd, int mode, uint32_t nx, uint32_t tiles) {
+    constexpr int S = SHIFT ? LINE : 0, LR = TR + S, H = TC / 2;
+    static_assert(TR % LINE == 0 && LR * H % NT == 0 && TR * TC % (2 * NT) == 0, "whole rounds of the workgroup");
+    __shared__ double tile[LR][TC + 1];
+    const int t = threadIdx.x;
+    for (uint32_t b = blockIdx.x; b < tiles; b += gridDim.x) {
+        const int64_t i0 = (int64_t)(b % nx) * TR - S, j0 = (int64_t)(b / nx) * TC;
+        auto shift = [&](const double *col) { return SHIFT ? (LINE - phase(col)) & (LINE - 1) : 0; };
+        if (i0 >= 0 && i0 + LR <= rows && j0 + TC <= cols) {
+            f64x2u v[LR * H / NT];
+#pragma unroll
+            for (int q = 0; q < LR * H / NT; ++q) {
+                const int e = t + NT * q, il = e / H, c2 = (e % H) * 2;
+                const f64x2u *p = reinterpret_cast<const f64x2u *>(src + (j0 + c2) + (i0 + il) * lds);
+                v[q] = SHIFT ? *p : __builtin_nontemporal_load(p);
+            }
+#pragma unroll
+            for (int q = 0; q < LR * H / NT; ++q) {
+                const int e = t + NT * q, il = e / H, c2 = (e % H) * 2;
+                tile[il][c2] = v[q].x;
+                tile[il][c2 + 1] = v[q].y;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < TR * TC / 2 / NT; ++q) {
+                const int e = t + NT * q, jl = e / (TR / 2);
+                double *col = dst + (j0 + jl) * ldd + i0;
+                const int r = (e % (TR / 2)) * 2 + shift(col);
+                f64x2u *d = reinterpret_cast<f64x2u *>(col + r);
+                const f64x2u old = mode == 2 ? *d : f64x2u{0.0, 0.0};
+                __builtin_nontemporal_store(combine2(f64x2u{tile[r][jl], tile[r + 1][jl]}, alpha, beta, old, mode), d);
+            }
+        } else {
+            for (int e = t; e < LR * TC; e += NT) {
+                const int il = e / TC, c = e % TC;
+                const int64_t i = i0 + il, j = j0 + c;
+                if (i >= 0 && i < rows && j < cols) tile[il][c] = src[j + i * lds];
+            }
+            __syncthreads();
+            for (int e = t; e < TR * TC; e += NT) {
+                const int jl = e / TR;
+                const int64_t j = j0 + jl;
+                if (j >= cols) break;
+                double *col = dst + j * ldd + i0;
+                const int r = e % TR + shift(col);
+                if (i0 + r >= 0 && i0 + r < rows) col[r] = combine(tile[r][jl], alpha, beta, col + r, mode);
+            }
+        }
+        __syncthreads();
+    }
+}
+
+template <int TR, int TC, bool SHIFT>
+void launch_transpose(int64_t rows, int64_t cols, double alpha, const double *src, int64_t lds, double beta,
+                      double *dst, int64_t ldd, int mode, hipStream_t s) {
+    const int64_t nx = (rows + (SHIFT ? LINE : 0) + TR - 1) / TR, tiles = nx * ((cols + TC - 1) / TC);
+    hipLaunchKernelGGL((transpose_kernel<TR, TC, SHIFT>), dim3((unsigned)std::min<int64_t>(tiles, 1 << 23)), dim3(NT),
+                       0, s, rows, cols, alpha, src, lds, beta, dst, ldd, mode, (uint32_t)nx, (uint32_t)tiles);
+}
+
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+inline int phase_of(const void *p) { return (int)(reinterpret_cast<uintptr_t>(p) & (8 * LINE - 1)); }   // bytes into its line
+
+int mode_of(double alpha, double beta) { return (alpha == 1.0 && beta == 0.0) ? 0 : (beta == 0.0 ? 1 : 2); }
 
 }  // namespace
 
@@ -195,18 +348,41 @@ int launch_block_transform(char op, int64_t rows, int64_t cols, double alpha,
                            const double *src, int64_t lds, double beta,
                            double *dst, int64_t ldd, hipStream_t s) {
     if (rows == 0 || cols == 0) return COSMA_AMD_OK;
-    const int mode = (alpha == 1.0 && beta == 0.0) ? 0 : (beta == 0.0 ? 1 : 2);
+    const int mode = mode_of(alpha, beta);
+    const bool in_phase = ldd % LINE == 0 && phase_of(dst) == 0;   // every column of dst starts at a line
+    const bool src_in_phase = lds % LINE == 0 && phase_of(src) == 0;
+    // src and dst together exceed the 256 MB last-level cache, which hides
+    // shared lines (8191 x 12289 'T': 421 us, in shifted windows 298 us, 5000 x
+    // 5001: 111 and 79 us, but 3000 x 5000: 46 and 53 us)
+    const bool large = rows * cols >= 20000000;
     if (op == 'N') {
-        const int vec = aligned16(src) && aligned16(dst) && (lds % 2 == 0) && (ldd % 2 == 0);
-        const int64_t pairs = (rows + 1) / 2;
-        const int64_t bx = (pairs + 255) / 256;
-        const int64_t by = std::min<int64_t>((cols + 1) / 2, 65535);
+        // a 512-row window would leave most threads idle (40 x 100000: 25 -> 15 us)
+        if (rows <= NT && rows * cols >= (1 << 20) && rows * cols <= (1 << 26)) {
+            const CopyBlock one{src, dst, lds, ldd, rows, cols};
+            return launch_block_copies(&one, 1, alpha, beta, s);
+        }
+        const bool shift = !in_phase && rows >= 1024, stream = rows * cols >= (1 << 24);
+        const int64_t bx = (rows + (shift ? LINE - 1 : 0) + 2 * NT - 1) / (2 * NT);
+        const int64_t by = std::min<int64_t>(stream ? cols : (cols + 1) / 2, 65535);
         if (bx > 0x7fffffffLL) {
             set_error("block_transform: %lld rows exceed the grid limit", (long long)rows);
             return COSMA_AMD_ERR_UNSUPPORTED;
         }
-        hipLaunchKernelGGL(copy_kernel, dim3((unsigned)bx, (unsigned)by), dim3(256), 0, s,
-                           rows, cols, alpha, src, lds, beta, dst, ldd, mode, vec);
+        const dim3 grid((unsigned)bx, (unsigned)by);
+#define CA_COPY(SHIFT, STREAM)                                                                                       \
+    hipLaunchKernelGGL((copy_kernel<SHIFT, STREAM>), grid, dim3(NT), 0, s, rows, cols, alpha, src, lds, beta, dst, \
+                       ldd, mode)
+        if (shift && stream) CA_COPY(true, true);
+        else if (shift) CA_COPY(true, false);
+        else if (stream) CA_COPY(false, true);
+        else CA_COPY(false, false);
+#undef CA_COPY
+    } else if (in_phase && src_in_phase && rows >= 4096 && rows * cols >= ((int64_t)1 << 26)) {
+        // both sides in whole lines (16384^2: 769 us in 64 x 64 tiles, 700 us;
+        // slower below 4096 rows, 2000 x 16000: 90 and 112 us)
+        launch_transpose<128, 64, false>(rows, cols, alpha, src, lds, beta, dst, ldd, mode, s);
+    } else if (!(in_phase && src_in_phase) && large && rows >= 1024 && cols >= 1024) {
+        launch_transpose<112, 64, true>(rows, cols, alpha, src, lds, beta, dst, ldd, mode, s);
     } else {
         const int64_t bx = (rows + TT - 1) / TT;
         int64_t by = (cols + TT - 1) / TT;
@@ -220,14 +396,44 @@ int launch_block_transform(char op, int64_t rows, int64_t cols, double alpha,
         // prefetches the next tile of a workgroup during the current one)
         if (vec && bx * by > 4096) by = (by + 3) / 4;
         if (vec)
-            hipLaunchKernelGGL(transpose_vec_kernel, dim3((unsigned)bx, (unsigned)by), dim3(TNT), 0, s,
+            hipLaunchKernelGGL(transpose_cached_vec_kernel, dim3((unsigned)bx, (unsigned)by), dim3(NT), 0, s,
                                rows, cols, alpha, src, lds, beta, dst, ldd, mode);
         else
-            hipLaunchKernelGGL(transpose_kernel, dim3((unsigned)bx, (unsigned)by), dim3(TNT), 0, s,
+            hipLaunchKernelGGL(transpose_cached_kernel, dim3((unsigned)bx, (unsigned)by), dim3(NT), 0, s,
                                rows, cols, alpha, src, lds, beta, dst, ldd, mode);
     }
     CA_HIP(hipGetLastError());
     return COSMA_AMD_OK;
+}
+
+int launch_block_copies(const CopyBlock *blocks, int64_t n, double alpha, double beta, hipStream_t s) {
+    const int mode = mode_of(alpha, beta);
+    BlockList list;
+    list.n = 0;
+    uint32_t groups = 0;
+    auto flush = [&]() -> int {
+        if (list.n == 0) return COSMA_AMD_OK;
+        hipLaunchKernelGGL(copy_list_kernel, dim3(groups), dim3(NT), 0, s, list, alpha, beta, mode);
+        CA_HIP(hipGetLastError());
+        list.n = 0;
+        groups = 0;
+        return COSMA_AMD_OK;
+    };
+    int rc;
+    for (int64_t i = 0; i < n; ++i) {
+        const CopyBlock &b = blocks[i];
+        if (b.rows == 0 || b.cols == 0) continue;
+        const int64_t pairs = (b.rows + LINE) / 2, total = pairs * b.cols;
+        if (b.rows > (1 << 26) || b.cols > (1 << 26) || total > (1 << 26)) {   // 1 GiB fills the chip by itself
+            rc = launch_block_transform('N', b.rows, b.cols, alpha, b.src, b.lds, beta, b.dst, b.ldd, s);
+            if (rc) return rc;
+            continue;
+        }
+        list.b[list.n++] = {b.src, b.dst, b.lds, b.ldd, (int)b.rows, (int)b.cols, groups, (uint32_t)pairs};
+        groups += (uint32_t)((total + NT * ITEMS - 1) / (NT * ITEMS));
+        if (list.n == LIST && (rc = flush())) return rc;
+    }
+    return flush();
 }
 
 }  // namespace cosma_amd
