@@ -688,20 +688,32 @@ int check_tiling(const char *name, const cosma_amd_block *blk, int64_t nb, int64
 
 // Gathers the blocks of one operand into the column-major device matrix dst
 // (leading dimension ld): host blocks are uploaded on h2d, device blocks are
-// copied by the block-copy kernel on stream s.
-int gather_blocks(cosma_amd_handle_t h, const cosma_amd_block *blk, int64_t nb, double *dst, int64_t ld,
-                  hipStream_t s) {
-    for (int64_t i = 0; i < nb; ++i) {
+// copied together on stream s (one launch per block made the 750 launches of
+// a 4000^3 product in 256 x 256 blocks take half of its 4.5 ms).
+int gather_blocks(cosma_amd_handle_t h, const cosma_amd_block *blk, const std::vector<Kind> &kinds, double *dst,
+                  int64_t ld, hipStream_t s) {
+    std::vector<CopyBlock> copies;
+    for (size_t i = 0; i < kinds.size(); ++i) {
         const cosma_amd_block &b = blk[i];
         if (b.rows == 0 || b.cols == 0) continue;
         const double *src = static_cast<const double *>(b.data);
         double *d = dst + b.row + b.col * ld;
-        const Kind kind = classify(src);
-        int rc = (kind == DEVICE) ? launch_block_transform('N', b.rows, b.cols, 1.0, src, b.ld, 0.0, d, ld, s)
-                                  : upload(h, d, ld, src, b.ld, b.rows, b.cols, kind);
-        if (rc) return rc;
+        if (kinds[i] == DEVICE) {
+            copies.push_back({src, d, b.ld, ld, b.rows, b.cols});
+        } else {
+            const int rc = upload(h, d, ld, src, b.ld, b.rows, b.cols, kinds[i]);
+            if (rc) return rc;
+        }
     }
-    return COSMA_AMD_OK;
+    return launch_block_copies(copies.data(), (int64_t)copies.size(), 1.0, 0.0, s);
+}
+
+// The kind of every non-empty block.
+std::vector<Kind> classify_blocks(const cosma_amd_block *blk, int64_t nb) {
+    std::vector<Kind> kinds((size_t)nb, PAGEABLE);
+    for (int64_t i = 0; i < nb; ++i)
+        if (blk[i].rows > 0 && blk[i].cols > 0) kinds[(size_t)i] = classify(blk[i].data);
+    return kinds;
 }
 
 }  // namespace
@@ -726,7 +738,8 @@ static int layout_dgemm_body(cosma_amd_handle_t h, char ta, char tb, int64_t m, 
 
     // ---- device copies: A, B as stored, X = op(A) op(B), staging for host C blocks
     bool host_c = false;
-    for (int64_t i = 0; i < nc; ++i) host_c |= (C[i].rows > 0 && C[i].cols > 0 && classify(C[i].data) != DEVICE);
+    const std::vector<Kind> kinds_c = classify_blocks(C, nc);
+    for (int64_t i = 0; i < nc; ++i) host_c |= (C[i].rows > 0 && C[i].cols > 0 && kinds_c[i] != DEVICE);
     const size_t needA = scale_only ? 0 : (size_t)arows * acols * 8, needB = scale_only ? 0 : (size_t)brows * bcols * 8;
     const size_t needX = (size_t)m * n * 8, needC = host_c ? needX : 0;
     size_t free_b = 0, total_b = 0;
@@ -752,7 +765,7 @@ static int layout_dgemm_body(cosma_amd_handle_t h, char ta, char tb, int64_t m, 
         for (int64_t i = 0; i < nc; ++i) {
             const cosma_amd_block &b = C[i];
             if (b.rows == 0 || b.cols == 0) continue;
-            const Kind kind = classify(b.data);
+            const Kind kind = kinds_c[i];
             if (kind == DEVICE) continue;
             rc = upload(h, dC + b.row + b.col * m, m, static_cast<const double *>(b.data), b.ld, b.rows, b.cols, kind);
             if (rc) return rc;
@@ -766,8 +779,8 @@ static int layout_dgemm_body(cosma_amd_handle_t h, char ta, char tb, int64_t m, 
     } else {
         if ((rc = grow(h->dA, needA)) || (rc = grow(h->dB, needB))) return rc;
         double *dA = static_cast<double *>(h->dA.ptr), *dB = static_cast<double *>(h->dB.ptr);
-        if ((rc = gather_blocks(h, A, na, dA, arows, s))) return rc;
-        if ((rc = gather_blocks(h, B, nb, dB, brows, s))) return rc;
+        if ((rc = gather_blocks(h, A, classify_blocks(A, na), dA, arows, s))) return rc;
+        if ((rc = gather_blocks(h, B, classify_blocks(B, nb), dB, brows, s))) return rc;
         hipEvent_t up;
         if ((rc = record(h, h->h2d, &up))) return rc;
         CA_HIP(hipStreamWaitEvent(s, up, 0));
@@ -780,18 +793,15 @@ static int layout_dgemm_body(cosma_amd_handle_t h, char ta, char tb, int64_t m, 
     }
 
     // ---- epilogue per C block: C_blk <- alpha * X_blk + beta * C_blk
+    std::vector<CopyBlock> updates;
     for (int64_t i = 0; i < nc; ++i) {
         const cosma_amd_block &b = C[i];
         if (b.rows == 0 || b.cols == 0) continue;
         const double *x = dX + b.row + b.col * m;
-        if (classify(b.data) == DEVICE) {
-            rc = launch_block_transform('N', b.rows, b.cols, alpha, x, m, beta, static_cast<double *>(b.data),
-                                        b.ld, s);
-        } else {
-            rc = launch_block_transform('N', b.rows, b.cols, alpha, x, m, beta, dC + b.row + b.col * m, m, s);
-        }
-        if (rc) return rc;
+        if (kinds_c[i] == DEVICE) updates.push_back({x, static_cast<double *>(b.data), m, b.ld, b.rows, b.cols});
+        else updates.push_back({x, dC + b.row + b.col * m, m, m, b.rows, b.cols});
     }
+    if ((rc = launch_block_copies(updates.data(), (int64_t)updates.size(), alpha, beta, s))) return rc;
     if (host_c) {
         hipEvent_t done;
         if ((rc = record(h, s, &done))) return rc;
@@ -799,7 +809,7 @@ static int layout_dgemm_body(cosma_amd_handle_t h, char ta, char tb, int64_t m, 
         for (int64_t i = 0; i < nc; ++i) {
             const cosma_amd_block &b = C[i];
             if (b.rows == 0 || b.cols == 0) continue;
-            const Kind kind = classify(b.data);
+            const Kind kind = kinds_c[i];
             if (kind == DEVICE) continue;
             rc = download(h, static_cast<double *>(b.data), b.ld, dC + b.row + b.col * m, m, b.rows, b.cols, kind);
             if (rc) return rc;
