@@ -121,8 +121,11 @@ int grouped_tile_shape(int cfg, int *bm, int *bn);
 int grouped_problem_flags(char ta, char tb, int64_t m, int64_t n, const double *a, int64_t lda, const double *b,
                           int64_t ldb, const double *c, int64_t ldc, int *flags, int *vec_c);
 // probs: nprob descriptors in device memory, sorted as planned, followed by
-// their nprob int64 tile_start values (the kernels search that array).
-int launch_grouped(int cfg, const GroupedProblem *probs, int nprob, int64_t total_tiles, int grid, hipStream_t s);
+// their nprob int64 tile_start values and the int owner of every tile.
+// dl: -1 if a problem is beyond the direct-LDS kernels' limits (dl_fits), else
+// the transposes (flags & 3) that all problems share, or 4.
+int launch_grouped(int cfg, const GroupedProblem *probs, int nprob, int64_t total_tiles, int grid, int dl,
+                   hipStream_t s);
 int grouped_create(cosma_amd_handle_t h, const cosma_amd_gemm_desc *d, int64_t count, int tile_config,
                    cosma_amd_grouped_t *out);
 int grouped_ozaki_create(cosma_amd_handle_t h, const cosma_amd_gemm_desc *d, int64_t count, int moduli,

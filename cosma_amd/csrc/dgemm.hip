@@ -534,21 +534,6 @@ __device__ __forceinline__ void direct_tile(const GroupedProblem &q, int64_t m0,
     }
 }
 
-// Grouped launches walk virtual tile ids v = blockIdx.x + i * gridDim.x; the
-// hardware places workgroup b on XCD b % 8.  Consecutive tiles (of one
-// problem, which share A and B panels) are kept on one XCD and its L2 by
-// handing out chunks of GROUP_CHUNK consecutive tiles: XCD x takes chunks x,
-// x + 8, x + 16, ... in dispatch order, so the decreasing-cost order of the
-// problems is kept at chunk granularity.  Bijective on [0, T): ids beyond
-// the last whole round of 8 chunks map to themselves.
-constexpr int64_t GROUP_CHUNK = 8;
-__device__ __forceinline__ int64_t grouped_tile_of(int64_t v, int64_t T) {
-    constexpr int64_t span = NXCD * GROUP_CHUNK;
-    if (v >= T / span * span) return v;
-    const int64_t xcd = v % NXCD, local = v / NXCD;
-    return ((local / GROUP_CHUNK) * NXCD + xcd) * GROUP_CHUNK + local % GROUP_CHUNK;
-}
-
 // The descriptor array is followed by the problems' first tile indices
 // (int64, same order): the binary search for a tile's problem walks this
 // compact array (8 bytes per problem, so its upper levels stay in the scalar
@@ -644,7 +629,8 @@ int launch_cfg(char ta, char tb, int64_t m, int64_t n, int64_t k, double alpha,
 }
 
 // ------------------------------------------------------------ grouped GEMM
-// One persistent launch over the tiles of many independent problems.  Tiles
+// One launch over the tiles of many independent problems, for plans beyond the
+// direct-LDS kernels' limits (dgemm_dl_grouped_kernel takes all others).  Tiles
 // are numbered problem by problem (problems in the order of the descriptor
 // array, which the host sorts by decreasing cost) and column-major inside a
 // problem; workgroup w takes the virtual ids w, w + G, w + 2G, ... mapped to
@@ -770,8 +756,10 @@ int grouped_problem_flags(char ta, char tb, int64_t m, int64_t n, const double *
     return COSMA_AMD_OK;
 }
 
-int launch_grouped(int cfg, const GroupedProblem *probs, int nprob, int64_t total_tiles, int grid, hipStream_t s) {
+int launch_grouped(int cfg, const GroupedProblem *probs, int nprob, int64_t total_tiles, int grid, int dl,
+                   hipStream_t s) {
     if (nprob == 0 || total_tiles == 0) return COSMA_AMD_OK;
+    if (dl >= 0 && cfg != 4) return launch_grouped_dl(cfg, probs, nprob, total_tiles, grid, dl, s);
     const dim3 g((unsigned)grid), b(NT);
     switch (cfg) {
     case 1: hipLaunchKernelGGL((dgemm_grouped_kernel<64, 64>), g, b, 0, s, probs, nprob, total_tiles); break;

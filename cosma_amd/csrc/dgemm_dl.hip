@@ -120,9 +120,10 @@ struct Operand {
     }
 };
 
-// Fragment reads of one operand: row base + 16 i, lane group g, sub-step ks
-// (k-pair kp = 4 ks + g).
-template <int R, bool KCONTIG>
+// Fragment reads of one operand: row rbase + 16 i, lane group g, sub-step ks
+// (k-pair kp = 4 ks + g).  Several blocks per wave (COUNT > 1) start at a
+// multiple of 32 rows.
+template <int R, bool KCONTIG, int COUNT>
 struct Frag {
     int o0, o1;
     __device__ __forceinline__ Frag(int rbase, int g) {
@@ -131,7 +132,7 @@ struct Frag {
             o1 = 2 * (rbase * 8 + ((g + 4) ^ row_swz(rbase)));
         } else {
             const int gb = 16 * (g & 1);
-            o0 = 2 * g * R + (R == 32 ? rbase ^ gb : rbase + gb);   // even i
+            o0 = 2 * g * R + (COUNT == 1 ? rbase ^ gb : rbase + gb);   // even i
             o1 = 2 * g * R + rbase - gb;                            // odd i
         }
     }
@@ -142,37 +143,26 @@ struct Frag {
     }
 };
 
-// NS: LDS stages; WPE: waves per SIMD (= workgroups per CU) it is built for.
-template <int BM, int BN, int NS, int WPE, bool AK, bool BKC>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void dgemm_dl_kernel(
-    int64_t M, int64_t N, int64_t K, double alpha,
-    const double *__restrict__ A, int64_t lda,
-    const double *__restrict__ B, int64_t ldb,
-    double beta, double *__restrict__ C, int64_t ldc, int group_m) {
+// One BM x BN tile of C at (m0, n0) with NS LDS stages in sm.  EDGE: the MFMAs
+// of 16 x 16 blocks that lie wholly outside C are skipped.
+template <int BM, int BN, int NS, bool AK, bool BKC, bool EDGE>
+__device__ __forceinline__ void dl_tile(int64_t M, int64_t N, int64_t K, double alpha, const double *__restrict__ A,
+                                        int64_t lda, const double *__restrict__ B, int64_t ldb, double beta,
+                                        double *__restrict__ C, int64_t ldc, int64_t m0, int64_t n0, double *sm) {
     using OA = Operand<BM, AK>;
     using OB = Operand<BN, BKC>;
     constexpr int STAGE = OA::SIZE + OB::SIZE;
     constexpr int LOADS = OA::LOADS + OB::LOADS;
     constexpr int FM = BM / 32, FN = BN / 32;
     constexpr bool EARLY_TAIL = BM * BN <= 64 * 64;
-    __shared__ __attribute__((aligned(16))) double sm[NS * STAGE];
-
-    // ---- tile rasterisation (XCD-aware, grouped along m)
-    const uint32_t tiles_m = (uint32_t)((M + BM - 1) / BM), tiles_n = (uint32_t)((N + BN - 1) / BN);
-    const uint32_t T = gridDim.x, q8 = T / NXCD, r8 = T % NXCD, xcd = blockIdx.x % NXCD, loc = blockIdx.x / NXCD;
-    const uint32_t bid = xcd * q8 + min(xcd, r8) + loc;
-    const uint32_t per_group = group_m * tiles_n, grp = bid / per_group, in_group = bid - grp * per_group;
-    const uint32_t gsize = min((uint32_t)group_m, tiles_m - grp * group_m);
-    const int64_t m0 = (int64_t)(grp * group_m + in_group % gsize) * BM;
-    const int64_t n0 = (int64_t)(in_group / gsize) * BN;
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave & 1, wn = wave >> 1;
     const int g = lane >> 4, li = lane & 15;
     const OA oa(A, lda, m0, M, wave, lane);
     const OB ob(B, ldb, n0, N, wave, lane);
-    const Frag<BM, AK> fra(wm * (BM / 2) + 4 * (li & 3) + (li >> 2), g);
-    const Frag<BN, BKC> frb(wn * (BN / 2) + li, g);
+    const Frag<BM, AK, FM> fra(wm * (BM / 2) + 4 * (li & 3) + (li >> 2), g);
+    const Frag<BN, BKC, FN> frb(wn * (BN / 2) + li, g);
 
     // Full steps; a row-contiguous operand with an odd extent keeps the last
     // k out of them (the 16-byte load of its last row reads one element
@@ -198,17 +188,21 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
 #pragma unroll
         for (int j = 0; j < FN; ++j) bf[ks][j] = frb.read(tile + OA::SIZE, j, ks);
     };
+    const int rows_in = EDGE ? (int)min((int64_t)FM, (M - m0 - wm * (BM / 2) + 15) >> 4) : FM;   // may be <= 0
+    const int cols_in = EDGE ? (int)min((int64_t)FN, (N - n0 - wn * (BN / 2) + 15) >> 4) : FN;
     auto mfmas = [&](int h) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
             for (int j = 0; j < FN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[h][i].x, bf[h][j].x, acc[i][j], 0, 0, 0);
+                if (!EDGE || (i < rows_in && j < cols_in))
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[h][i].x, bf[h][j].x, acc[i][j], 0, 0, 0);
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
             for (int j = 0; j < FN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[h][i].y, bf[h][j].y, acc[i][j], 0, 0, 0);
+                if (!EDGE || (i < rows_in && j < cols_in))
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[h][i].y, bf[h][j].y, acc[i][j], 0, 0, 0);
     };
     auto issue = [&](int kt_, double *tile) {
         oa.issue(kt_ * BK, tile, wave);
@@ -260,9 +254,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
         OB::tail_store(sm + OA::SIZE, tb);
         __syncthreads();
         read_frags(sm, 0);
-        read_frags(sm, 1);
+        if (kt > BK / 2) read_frags(sm, 1);
         mfmas(0);
-        mfmas(1);
+        if (kt > BK / 2) mfmas(1);
     }
     __builtin_amdgcn_s_waitcnt(wait_vm(0));   // no LDS writes outstanding at exit
 
@@ -299,6 +293,63 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
                 }
             }
         }
+    }
+}
+
+// NS: LDS stages; WPE: waves per SIMD (= workgroups per CU) it is built for.
+template <int BM, int BN, int NS, int WPE, bool AK, bool BKC>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void dgemm_dl_kernel(
+    int64_t M, int64_t N, int64_t K, double alpha,
+    const double *__restrict__ A, int64_t lda,
+    const double *__restrict__ B, int64_t ldb,
+    double beta, double *__restrict__ C, int64_t ldc, int group_m) {
+    __shared__ __attribute__((aligned(16))) double sm[NS * (BM + BN) * BK];
+    // ---- tile rasterisation (XCD-aware, grouped along m)
+    const uint32_t tiles_m = (uint32_t)((M + BM - 1) / BM), tiles_n = (uint32_t)((N + BN - 1) / BN);
+    const uint32_t T = gridDim.x, q8 = T / NXCD, r8 = T % NXCD, xcd = blockIdx.x % NXCD, loc = blockIdx.x / NXCD;
+    const uint32_t bid = xcd * q8 + min(xcd, r8) + loc;
+    const uint32_t per_group = group_m * tiles_n, grp = bid / per_group, in_group = bid - grp * per_group;
+    const uint32_t gsize = min((uint32_t)group_m, tiles_m - grp * group_m);
+    const int64_t m0 = (int64_t)(grp * group_m + in_group % gsize) * BM;
+    const int64_t n0 = (int64_t)(in_group / gsize) * BN;
+    dl_tile<BM, BN, NS, AK, BKC, false>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, m0, n0, sm);
+}
+
+// Grouped tiles: workgroup w takes the virtual ids w, w + G, ... of all
+// problems' tiles, mapped to tiles by grouped_tile_of.  TRANS: the problems'
+// common transposes (GroupedProblem::flags), or MIXED, whose four loops in one
+// kernel need registers for three workgroups per CU in place of four.
+// What bounds it: a tile takes about 1.9 us of its CU before and after its
+// k-steps (owner, descriptor and first loads in a chain, C's stores), as much
+// as four 64 x 64 steps, and the batch's 2 GB from HBM take 0.4 ms; one
+// workgroup per tile overlaps these best.  4096 NN products, m, n, k log-uniform
+// in [16, 512], tuned: 889 us register-staged with a search for the owner,
+// 728 us here, 690 us with the blocks outside C skipped and the kernel of one
+// transpose.  Cutting a tile into four rows or columns of blocks, whichever
+// balances its waves better at an edge, spilled and lost (774 us).
+constexpr int MIXED = 4;
+template <int BM, int BN, int NS, int WPE, int TRANS>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void dgemm_dl_grouped_kernel(
+    const GroupedProblem *__restrict__ probs, const int *__restrict__ owner, int64_t total_tiles) {
+    __shared__ __attribute__((aligned(16))) double sm[NS * (BM + BN) * BK];
+    for (int64_t v = blockIdx.x; v < total_tiles; v += gridDim.x) {
+        const int64_t t = grouped_tile_of(v, total_tiles);
+        const GroupedProblem &q = probs[owner[t]];
+        const uint32_t local = (uint32_t)(t - q.tile_start), tiles_m = (uint32_t)((q.m + BM - 1) / BM);
+        const int64_t m0 = (int64_t)(local % tiles_m) * BM, n0 = (int64_t)(local / tiles_m) * BN;
+        const bool scale_only = (q.k == 0 || q.alpha == 0.0);
+        const int64_t K = scale_only ? 0 : q.k;
+        const double alpha = scale_only ? 0.0 : q.alpha;
+        if (v >= gridDim.x) __syncthreads();   // the previous tile's last LDS reads are done
+#define CA_TILE(X, Y)                                                                                           \
+    dl_tile<BM, BN, NS, X, Y, true>(q.m, q.n, K, alpha, q.a, q.lda, q.b, q.ldb, q.beta, q.c, q.ldc, m0, n0, sm)
+        switch (TRANS == MIXED ? q.flags & 3 : TRANS) {   // bit 0: A transposed, bit 1: B transposed
+        case 0: CA_TILE(false, true); break;
+        case 1: CA_TILE(true, true); break;
+        case 2: CA_TILE(false, false); break;
+        default: CA_TILE(true, false); break;
+        }
+#undef CA_TILE
     }
 }
 
@@ -382,6 +433,31 @@ int launch_dl(DlTile tile, char ta, char tb, int64_t m, int64_t n, int64_t k, do
     default: CA_DL(32, 32, 4, 4); break;
     }
 #undef CA_DL
+    CA_HIP(hipGetLastError());
+    return COSMA_AMD_OK;
+}
+
+int launch_grouped_dl(int cfg, const GroupedProblem *probs, int nprob, int64_t total_tiles, int grid, int trans,
+                      hipStream_t s) {
+    const int *owner = reinterpret_cast<const int *>(reinterpret_cast<const int64_t *>(probs + nprob) + nprob);
+    const dim3 g((unsigned)grid), b(NT);
+#define CA_GROUPED(BM, BN, NS, WPE, TRANS) \
+    hipLaunchKernelGGL((dgemm_dl_grouped_kernel<BM, BN, NS, WPE, TRANS>), g, b, 0, s, probs, owner, total_tiles)
+    switch (cfg) {
+    case 1:
+        switch (trans) {
+        case 0: CA_GROUPED(64, 64, 2, 4, 0); break;
+        case 1: CA_GROUPED(64, 64, 2, 4, 1); break;
+        case 2: CA_GROUPED(64, 64, 2, 4, 2); break;
+        case 3: CA_GROUPED(64, 64, 2, 4, 3); break;
+        default: CA_GROUPED(64, 64, 2, 3, MIXED); break;
+        }
+        break;
+    case 2: CA_GROUPED(128, 64, 2, 2, MIXED); break;
+    case 3: CA_GROUPED(128, 128, 2, 2, MIXED); break;
+    default: CA_GROUPED(32, 32, 2, 6, MIXED); break;
+    }
+#undef CA_GROUPED
     CA_HIP(hipGetLastError());
     return COSMA_AMD_OK;
 }

@@ -13,7 +13,7 @@
 // with no allocation, no memset and no host synchronisation, so it can be
 // captured; cosma_amd_grouped_graph_run captures it once into a hipGraph and
 // replays that.  The tuner times every tile configuration (LDS-staged 64x64,
-// 128x64, 128x128; direct 64x64 and 32x32) with persistent grids of 1, 2, 4
+// 128x64, 128x128, 32x32; direct 64x64) with persistent grids of 1, 2, 4
 // and 8 workgroups per CU and one workgroup per tile, keeps the fastest, and
 // remembers it process-wide for plans with the same problem shapes.
 #include <algorithm>
@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "dgemm_dl.hpp"
 
 struct cosma_amd_grouped_s {
     cosma_amd_handle_t h = nullptr;
@@ -34,6 +35,7 @@ struct cosma_amd_grouped_s {
     int64_t total_tiles[6] = {0, 0, 0, 0, 0, 0};
     int cfg = 1;
     int grid = 1;
+    int dl = -1;      // launch_grouped's
     hipStream_t capture = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -130,6 +132,12 @@ int grouped_create(cosma_amd_handle_t h, const cosma_amd_gemm_desc *d, int64_t c
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost[x] > cost[y]; });
 
     auto p = new cosma_amd_grouped_s();
+    if (std::all_of(probs.begin(), probs.end(),
+                    [](const GroupedProblem &g) { return dl_fits(g.m, g.n, g.k, g.lda, g.ldb); })) {
+        p->dl = probs.empty() ? 4 : probs[0].flags & 3;
+        for (const GroupedProblem &g : probs)
+            if ((g.flags & 3) != p->dl) p->dl = 4;
+    }
     p->h = h;
     p->nprob = (int)probs.size();
     p->signature = fnv(sig, (uint64_t)probs.size());
@@ -152,8 +160,14 @@ int grouped_create(cosma_amd_handle_t h, const cosma_amd_gemm_desc *d, int64_t c
         // descriptors, then their first tile indices (the kernels' search array)
         std::vector<int64_t> starts;
         for (const GroupedProblem &g : sorted) starts.push_back(g.tile_start);
+        // and the owner of every tile
+        std::vector<int> owner;
+        owner.reserve((size_t)t);
+        for (size_t i = 0; i < sorted.size(); ++i)
+            owner.insert(owner.end(), (size_t)((i + 1 < sorted.size() ? starts[i + 1] : t) - starts[i]), (int)i);
         const size_t dbytes = sorted.size() * sizeof(GroupedProblem), sbytes = starts.size() * sizeof(int64_t);
-        hipError_t e = dev_alloc(reinterpret_cast<void **>(&p->dev[cfg]), dbytes + sbytes);
+        const size_t obytes = owner.size() * sizeof(int);
+        hipError_t e = dev_alloc(reinterpret_cast<void **>(&p->dev[cfg]), dbytes + sbytes + obytes);
         if (e != hipSuccess) {
             (void)hipGetLastError();
             set_error("grouped dgemm: descriptor allocation failed (%s)", hipGetErrorString(e));
@@ -163,6 +177,8 @@ int grouped_create(cosma_amd_handle_t h, const cosma_amd_gemm_desc *d, int64_t c
         e = hipMemcpy(p->dev[cfg], sorted.data(), dbytes, hipMemcpyHostToDevice);
         if (e == hipSuccess)
             e = hipMemcpy(reinterpret_cast<char *>(p->dev[cfg]) + dbytes, starts.data(), sbytes, hipMemcpyHostToDevice);
+        if (e == hipSuccess)
+            e = hipMemcpy(reinterpret_cast<char *>(p->dev[cfg]) + dbytes + sbytes, owner.data(), obytes, hipMemcpyHostToDevice);
         if (e != hipSuccess) {
             set_error("grouped dgemm: descriptor upload failed (%s)", hipGetErrorString(e));
             rc = COSMA_AMD_ERR_HIP;
@@ -191,7 +207,7 @@ int grouped_create(cosma_amd_handle_t h, const cosma_amd_gemm_desc *d, int64_t c
 
 int grouped_run(cosma_amd_grouped_t p, hipStream_t s) {
     CA_HIP(hipSetDevice(p->h->device));
-    return launch_grouped(p->cfg, p->dev[p->cfg], p->nprob, p->total_tiles[p->cfg], p->grid, s);
+    return launch_grouped(p->cfg, p->dev[p->cfg], p->nprob, p->total_tiles[p->cfg], p->grid, p->dl, s);
 }
 
 int grouped_graph_run(cosma_amd_grouped_t p, hipStream_t s) {
@@ -233,9 +249,9 @@ int grouped_tune(cosma_amd_grouped_t p, hipStream_t s) {
         grids.erase(std::unique(grids.begin(), grids.end()), grids.end());
         for (int64_t g : grids) {
             if (g < 1) continue;
-            if ((rc = launch_grouped(cfg, p->dev[cfg], p->nprob, tiles, (int)g, s))) break;   // warm-up
+            if ((rc = launch_grouped(cfg, p->dev[cfg], p->nprob, tiles, (int)g, p->dl, s))) break;   // warm-up
             CA_HIP(hipEventRecord(a, s));
-            for (int r = 0; r < 3 && rc == COSMA_AMD_OK; ++r) rc = launch_grouped(cfg, p->dev[cfg], p->nprob, tiles, (int)g, s);
+            for (int r = 0; r < 3 && rc == COSMA_AMD_OK; ++r) rc = launch_grouped(cfg, p->dev[cfg], p->nprob, tiles, (int)g, p->dl, s);
             CA_HIP(hipEventRecord(b, s));
             CA_HIP(hipEventSynchronize(b));
             float ms = 0.0f;

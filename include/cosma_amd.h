@@ -238,10 +238,11 @@ int cosma_amd_handle_last_mode(cosma_amd_handle_t handle);
 
 /*
  * Selects the DGEMM tile shape for later cosma_amd_dgemm calls (process-wide):
- * tile_config 0 = automatic, 1 = 128x128, 2 = 256x128, 3 = 128x256 (m x n of
- * C per workgroup), 4 = the kernel with direct LDS loads (128x128, two
- * workgroups per CU; m and n multiples of 128, k of 16, 16-byte aligned
- * operands with even leading dimensions; other calls take the automatic
+ * tile_config 0 = automatic (the kernel with direct LDS loads in the tile
+ * expected fastest for the shape, 128x128 to 32x32), 1 = 128x128, 2 = 256x128,
+ * 3 = 128x256 (m x n of C per workgroup, register-staged), 4 = the kernel with
+ * direct LDS loads in 128x128 tiles (m and n multiples of 128, k of 16, 16-byte
+ * aligned operands with even leading dimensions; other calls take the automatic
  * choice); group_m = tile-rows walked before moving along n
  * (0 = default for the shape).  No counterpart in the reference (Tiled-MM's
  * tile sizes, COSMA_GPU_MAX_TILE_*, describe host streaming tiles, not
@@ -290,9 +291,9 @@ typedef struct cosma_amd_grouped_s *cosma_amd_grouped_t;
  * are dropped).  The descriptors are copied to the device; the operand
  * pointers must stay valid while the plan is used.  tile_config: 0 = the
  * tuned choice for these shapes if one exists in the process, else 64x64;
- * 1 = 64x64, 2 = 128x64, 3 = 128x128 C tiles staged through LDS by four
- * waves; 4 = 64x64 and 5 = 32x32 C tiles computed by one wave each with
- * fragments loaded straight from global memory (no LDS).
+ * 1 = 64x64, 2 = 128x64, 3 = 128x128, 5 = 32x32 C tiles staged through LDS by
+ * four waves; 4 = 64x64 C tiles computed by one wave each with fragments
+ * loaded straight from global memory (no LDS).
  * cosma_amd_grouped_run: one persistent kernel launch on `stream` (no
  * allocation, memset or synchronisation: capturable).
  * cosma_amd_grouped_graph_run: captures the launch into a hipGraph on first
