@@ -56,36 +56,66 @@ __global__ void clear_u64(unsigned long long *p, int64_t n) {
 // columns of op(B)): the max |x| of every vector (as bit patterns, for the
 // exponents), the sum of squares of every vector (for the bound on |A'B'|)
 // and, for every k, the sum of squares across the vectors (for the error
-// estimate).  No LDS: a wave reads 64 consecutive elements along the
-// contiguous dimension per load, keeps the reduction along the other
-// dimension in registers, and reduces across its lanes with shuffles.
-// CONTIG (element (r, k) at x[k + r * ld]): lane = k, wave = 64 vectors, one
-// wave max and sum per vector and STATS_KC * 64 k; otherwise (x[r + k * ld]):
-// lane = r within STATS_RCH chunks of 64 rows, wave = 64 k, one wave sum per
-// k.  Workgroups cover STATS_KC * 64 (CONTIG) or STATS_RCH * 64 lanes x
-// STATS_SPAN of the other dimension (4 waves x STATS_SPAN / 4).
-// The contiguous form reads with non-temporal loads (8192^2: 140 -> 128 us).
-constexpr int STATS_SPAN = 256;
+// estimate).  A wave reads 64 consecutive elements along the contiguous
+// dimension per load, keeps the reduction along the other dimension in
+// registers, and reduces across its lanes with shuffles.
+// CONTIG (element (r, k) at x[k + r * ld]): lane = k, one wave max and sum per
+// vector and STATS_KC * 64 k; otherwise (x[r + k * ld]): lane = r within
+// STATS_RCH chunks of 64 rows, one wave sum per k.  A workgroup covers STATS_KC
+// * 64 (CONTIG) or STATS_RCH * 64 lanes x `span` of the other dimension (4
+// waves x span / 4).
+// What bounds it: HBM reads, where there are workgroups enough and little else
+// to do.  The sums that the four waves share meet in LDS before the global
+// atomics, eight lane reductions go together (reduce8), the span shrinks with
+// the operand until the chip is filled, and the loads stream past the caches
+// (3000 x 4100, contiguous: 60 us in 108 workgroups, 22 us in 846; 8192^2: 133 us
+// -> 99 us = 5.4 TB/s, strided 141 -> 110 us, of which 25 us non-temporal loads).
 constexpr int STATS_KC = 8;   // 64-wide k chunks per workgroup (contiguous vectors)
 constexpr int STATS_RCH = 4;  // 64-row chunks per wave (strided vectors)
+constexpr int STATS_GROUPS = 512;   // workgroups that fill the chip
+constexpr int STATS_U = 8;    // vectors (k) per group of loads; spans are multiples of 4 * STATS_U
+
+// Reduces eight values per lane over the wave: the result of value lane & 7, in
+// every lane.  Each of the first three steps hands the values of the other
+// parity to the neighbour and keeps half as many: ten shuffles in place of 48.
+template <typename T, typename Op>
+__device__ __forceinline__ T reduce8(T (&v)[STATS_U], Op op) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int n = STATS_U / 2, bit = 1; n > 0; n >>= 1, bit <<= 1) {
+        const bool odd = (lane & bit) != 0;
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+            const T keep = odd ? v[2 * i + 1] : v[2 * i], give = odd ? v[2 * i] : v[2 * i + 1];
+            v[i] = op(keep, __shfl_xor(give, bit));
+        }
+    }
+    T r = v[0];
+#pragma unroll
+    for (int off = 8; off < 64; off <<= 1) r = op(r, __shfl_xor(r, off));
+    return r;
+}
 
 template <bool CONTIG>
 __global__ __launch_bounds__(256) void stats_kernel(const double *__restrict__ x, int64_t ld, int64_t R, int64_t K,
-                                                    unsigned long long *maxbits, double *ksq, double *rsq,
+                                                    int span, unsigned long long *maxbits, double *ksq, double *rsq,
                                                     double *rabs) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    constexpr int PER_WAVE = STATS_SPAN / 4, U = 8;
+    const int per_wave = span / 4;
+    constexpr int U = STATS_U;
+    const auto sum = [](double x, double y) { return x + y; };
+    const auto largest = [](unsigned long long x, unsigned long long y) { return x > y ? x : y; };
     if (CONTIG) {
-        // A workgroup covers STATS_KC chunks of 64 consecutive k; each lane
-        // accumulates its k of every chunk for a group of U vectors before
-        // the group's cross-lane reductions, so there is one reduction per
-        // STATS_KC * 64 elements of a vector (and 8 x 8 loads in flight).
+        // Each lane accumulates its k of every chunk for a group of U vectors
+        // before the group's cross-lane reductions, so there is one reduction
+        // per STATS_KC * 64 elements of a vector (and 8 x 8 loads in flight).
+        __shared__ double part[4][STATS_KC * 64];
         const int64_t kbase = (int64_t)blockIdx.x * 64 * STATS_KC + lane;
-        const int64_t rb = (int64_t)blockIdx.y * STATS_SPAN + wave * PER_WAVE;
+        const int64_t rb = (int64_t)blockIdx.y * span + wave * per_wave;
         double ss[STATS_KC];
 #pragma unroll
         for (int c = 0; c < STATS_KC; ++c) ss[c] = 0.0;
-        for (int q0 = 0; q0 < PER_WAVE; q0 += U) {
+        for (int q0 = 0; q0 < per_wave; q0 += U) {
             unsigned long long b[U];
             double q[U], l1[U];
 #pragma unroll
@@ -112,42 +142,32 @@ __global__ __launch_bounds__(256) void stats_kernel(const double *__restrict__ x
                     b[u] = bb > b[u] ? bb : b[u];
                 }
             }
-            // U independent lane reductions (max and sum of squares), stepped
-            // together so their shuffle latencies overlap
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const unsigned long long o = __shfl_xor(b[u], off);
-                    b[u] = o > b[u] ? o : b[u];
-                    q[u] += __shfl_xor(q[u], off);
-                    l1[u] += __shfl_xor(l1[u], off);
-                }
-            }
+            const unsigned long long mine = reduce8(b, largest);
+            const double qs = reduce8(q, sum), as = reduce8(l1, sum);
             if (lane < U && rb + q0 + lane < R) {
-                unsigned long long mine = b[0];
-                double qs = q[0], as = l1[0];
-#pragma unroll
-                for (int u = 1; u < U; ++u) {
-                    mine = lane == u ? b[u] : mine;
-                    qs = lane == u ? q[u] : qs;
-                    as = lane == u ? l1[u] : as;
-                }
                 atomicMax(&maxbits[rb + q0 + lane], mine);
                 atomicAdd(&rsq[rb + q0 + lane], qs);
                 atomicAdd(&rabs[rb + q0 + lane], as);
             }
         }
 #pragma unroll
-        for (int c = 0; c < STATS_KC; ++c)
-            if (kbase + 64 * c < K) atomicAdd(&ksq[kbase + 64 * c], ss[c]);
+        for (int c = 0; c < STATS_KC; ++c) part[wave][64 * c + lane] = ss[c];
+        __syncthreads();
+#pragma unroll
+        for (int c = wave; c < STATS_KC; c += 4) {
+            const int i = 64 * c + lane;
+            const double total = (part[0][i] + part[1][i]) + (part[2][i] + part[3][i]);
+            if (kbase + 64 * c < K) atomicAdd(&ksq[kbase + 64 * c], total);
+        }
     } else {
         // A wave covers STATS_RCH chunks of 64 rows (lane = row within a
-        // chunk) for PER_WAVE k: the per-k sums of squares accumulate over
+        // chunk) for per_wave k: the per-k sums of squares accumulate over
         // the chunks in the lane before one cross-lane reduction, and the
         // STATS_RCH * U loads of a group are all in flight together.
+        __shared__ unsigned long long pmax[4][STATS_RCH * 64];
+        __shared__ double psq[4][STATS_RCH * 64], pabs[4][STATS_RCH * 64];
         const int64_t rbase = (int64_t)blockIdx.x * 64 * STATS_RCH + lane;
-        const int64_t kb = (int64_t)blockIdx.y * STATS_SPAN + wave * PER_WAVE;
+        const int64_t kb = (int64_t)blockIdx.y * span + wave * per_wave;
         unsigned long long best[STATS_RCH];
         double rs[STATS_RCH], ra[STATS_RCH];
 #pragma unroll
@@ -156,7 +176,7 @@ __global__ __launch_bounds__(256) void stats_kernel(const double *__restrict__ x
             rs[c] = 0.0;
             ra[c] = 0.0;
         }
-        for (int q0 = 0; q0 < PER_WAVE; q0 += U) {
+        for (int q0 = 0; q0 < per_wave; q0 += U) {
             double v[STATS_RCH][U];
 #pragma unroll
             for (int c = 0; c < STATS_RCH; ++c) {
@@ -164,7 +184,7 @@ __global__ __launch_bounds__(256) void stats_kernel(const double *__restrict__ x
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const int64_t k = kb + q0 + u;
-                    v[c][u] = (r < R && k < K) ? x[r + k * ld] : 0.0;
+                    v[c][u] = (r < R && k < K) ? __builtin_nontemporal_load(x + r + k * ld) : 0.0;
                 }
             }
             double sq[U];
@@ -181,33 +201,40 @@ __global__ __launch_bounds__(256) void stats_kernel(const double *__restrict__ x
                     rs[c] += q;
                     ra[c] += fabs(v[c][u]);
                 }
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-                for (int u = 0; u < U; ++u) sq[u] += __shfl_xor(sq[u], off);
-            }
-            if (lane < U && kb + q0 + lane < K) {
-                double mine = sq[0];
-#pragma unroll
-                for (int u = 1; u < U; ++u) mine = lane == u ? sq[u] : mine;
-                atomicAdd(&ksq[kb + q0 + lane], mine);
-            }
+            const double mine = reduce8(sq, sum);
+            if (lane < U && kb + q0 + lane < K) atomicAdd(&ksq[kb + q0 + lane], mine);
         }
 #pragma unroll
         for (int c = 0; c < STATS_RCH; ++c) {
-            const int64_t r = rbase + 64 * c;
-            if (r < R) {
-                atomicMax(&maxbits[r], best[c]);
-                atomicAdd(&rsq[r], rs[c]);
-                atomicAdd(&rabs[r], ra[c]);
+            pmax[wave][64 * c + lane] = best[c];
+            psq[wave][64 * c + lane] = rs[c];
+            pabs[wave][64 * c + lane] = ra[c];
+        }
+        __syncthreads();
+        const int i = 64 * wave + lane;   // wave w adds up chunk w
+        const int64_t r = rbase + 64 * wave;
+        static_assert(STATS_RCH == 4, "one chunk of rows per wave");
+        if (r < R) {
+            unsigned long long m = 0;
+            double sq = 0.0, sa = 0.0;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                m = pmax[w][i] > m ? pmax[w][i] : m;
+                sq += psq[w][i];
+                sa += pabs[w][i];
             }
+            atomicMax(&maxbits[r], m);
+            atomicAdd(&rsq[r], sq);
+            atomicAdd(&rabs[r], sa);
         }
     }
 }
 
-__global__ void exponents_kernel(const unsigned long long *maxbits, int64_t R, int slices, int *E,
+// Exponents of both operands: n maxima (the padding rows between and after them
+// have a maximum of zero).
+__global__ void exponents_kernel(const unsigned long long *maxbits, int64_t n, int slices, int *E,
                                  int *nonfinite) {
-    for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < R; r += (int64_t)gridDim.x * blockDim.x) {
+    for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x) {
         const unsigned long long b = maxbits[r];
         if (b >= 0x7ff0000000000000ull) atomicOr(nonfinite, 1);   // inf or NaN
         E[r] = row_exponent(b, slices);
@@ -301,7 +328,8 @@ __global__ __launch_bounds__(256) void split_contig(SplitArgs a, int64_t Rpad) {
 // transposed through LDS (non-temporal loads).  Each k of the tile is one
 // 128-byte run of the 16 rows; each output row leaves as one 256-byte run
 // (16 lanes) per residue plane.
-// blockIdx.x -> 16 rows, blockIdx.y -> 256 k.
+// blockIdx.x -> 16 rows, blockIdx.y -> 256 k.  (32 rows, 256-byte runs, per
+// workgroup of 512: 8192^2 338 -> 389 us.)
 __global__ __launch_bounds__(256) void split_strided(SplitArgs a) {
     __shared__ double tile[256][17];
     const int t = threadIdx.x;
@@ -767,19 +795,25 @@ int ozaki_dgemm(cosma_amd_handle_t h, char ta, char tb, int64_t m, int64_t n, in
     int *E = reinterpret_cast<int *>(rabsB + Np + 1);
     int *F = E + Mp;
     double *nrm = reinterpret_cast<double *>(aux + norm_off);
-    hipLaunchKernelGGL(clear_u64, dim3(grid_for(nclear)), dim3(256), 0, s, maxA, nclear);
+    // everything up to and with the first pass's partial norms
+    const int64_t words = (int64_t)(norm_off / 8) + NORM_SLOTS;
+    hipLaunchKernelGGL(clear_u64, dim3(grid_for(words)), dim3(256), 0, s, maxA, words);
     const bool a_rows_contig = ta == 'T', b_rows_contig = tb == 'N';   // op rows contiguous in k
-    // grid: x over the contiguous dimension in 64s, y over the other in STATS_SPAN
-    auto stats_grid = [](int64_t R, int64_t K, bool contig) {
-        const int64_t fast = contig ? K : R, slow = contig ? R : K, span = 64 * (contig ? STATS_KC : STATS_RCH);
-        return dim3((unsigned)((fast + span - 1) / span), (unsigned)((slow + STATS_SPAN - 1) / STATS_SPAN));
+    auto stats = [&](const double *x, int64_t ld, int64_t R, bool contig, unsigned long long *mx, double *ks, double *rs,
+                     double *ra) {
+        // x over the contiguous dimension, y over the other in spans
+        const int64_t fast = contig ? k : R, slow = contig ? R : k, lanes = 64 * (contig ? STATS_KC : STATS_RCH);
+        const int64_t gx = (fast + lanes - 1) / lanes;
+        int span = 256;
+        while (span > 4 * STATS_U && gx * ((slow + span - 1) / span) < STATS_GROUPS) span /= 2;
+        const dim3 grid((unsigned)gx, (unsigned)((slow + span - 1) / span));
+        if (contig) hipLaunchKernelGGL(stats_kernel<true>, grid, dim3(256), 0, s, x, ld, R, k, span, mx, ks, rs, ra);
+        else hipLaunchKernelGGL(stats_kernel<false>, grid, dim3(256), 0, s, x, ld, R, k, span, mx, ks, rs, ra);
     };
-    if (a_rows_contig) hipLaunchKernelGGL(stats_kernel<true>, stats_grid(m, k, true), dim3(256), 0, s, a, lda, m, k, maxA, ksqA, rsqA, rabsA);
-    else hipLaunchKernelGGL(stats_kernel<false>, stats_grid(m, k, false), dim3(256), 0, s, a, lda, m, k, maxA, ksqA, rsqA, rabsA);
-    if (b_rows_contig) hipLaunchKernelGGL(stats_kernel<true>, stats_grid(n, k, true), dim3(256), 0, s, b, ldb, n, k, maxB, ksqB, rsqB, rabsB);
-    else hipLaunchKernelGGL(stats_kernel<false>, stats_grid(n, k, false), dim3(256), 0, s, b, ldb, n, k, maxB, ksqB, rsqB, rabsB);
-    hipLaunchKernelGGL(exponents_kernel, dim3(grid_for(m)), dim3(256), 0, s, maxA, m, slices, E, flag);
-    hipLaunchKernelGGL(exponents_kernel, dim3(grid_for(n)), dim3(256), 0, s, maxB, n, slices, F, flag);
+    stats(a, lda, m, a_rows_contig, maxA, ksqA, rsqA, rabsA);
+    stats(b, ldb, n, b_rows_contig, maxB, ksqB, rsqB, rabsB);
+    // maxA and maxB adjoin, and so do E and F
+    hipLaunchKernelGGL(exponents_kernel, dim3(grid_for(Mp + Np)), dim3(256), 0, s, maxA, Mp + Np, slices, E, flag);
     CA_HIP(hipGetLastError());
     // One read-back of the contiguous span ksqA .. F (each small copy costs
     // tens of microseconds of fixed overhead, which several copies paid in
@@ -962,8 +996,9 @@ int ozaki_dgemm(cosma_amd_handle_t h, char ta, char tb, int64_t m, int64_t n, in
         pr.out = out; pr.ldo = ldr;
         // ---- 4. recombination with the norm of X (beta == 0: C written in
         // the same pass; otherwise C stays untouched until the check)
-        hipLaunchKernelGGL(clear_u64, dim3(1), dim3(NORM_SLOTS), 0, s, reinterpret_cast<unsigned long long *>(nrm),
-                           (int64_t)NORM_SLOTS);
+        if (passes > 1)
+            hipLaunchKernelGGL(clear_u64, dim3(1), dim3(NORM_SLOTS), 0, s, reinterpret_cast<unsigned long long *>(nrm),
+                               (int64_t)NORM_SLOTS);
         const int mode = beta == 0.0 ? EPI_WRITE_NORM : EPI_NORM;
         CrtConst cc;
         const dim3 gcrt((unsigned)((m + 256 * CRT_ROWS - 1) / (256 * CRT_ROWS)), (unsigned)std::min<int64_t>(n, 65535));

@@ -11,6 +11,16 @@ namespace cosma_amd {
 inline constexpr int kModuli[20] = {256, 255, 253, 251, 247, 241, 239, 233, 229, 227,
                                     223, 217, 211, 199, 197, 193, 191, 181, 179, 173};
 constexpr int MAX_MODULI = 20;
+// Products of consecutive groups of moduli, each below 2^48.
+constexpr int MOD_GROUP = 6;
+constexpr double group_product(int first) {
+    double p = 1.0;
+    for (int l = first; l < first + MOD_GROUP && l < MAX_MODULI; ++l) p *= kModuli[l];
+    return p;
+}
+constexpr double kGroupProduct[4] = {group_product(0), group_product(6), group_product(12), group_product(18)};
+constexpr double kGroupInverse[4] = {1.0 / kGroupProduct[0], 1.0 / kGroupProduct[1], 1.0 / kGroupProduct[2],
+                                     1.0 / kGroupProduct[3]};
 // CRT limbs: 4 limbs of 41 bits cover M < 2^164 (20 moduli: M ~ 2^155.4), and a
 // limb sum of 20 terms |c_l| * w < 20 * 2^7 * 2^41 < 2^53 stays exact in FP64.
 constexpr int LIMB = 41;
@@ -100,32 +110,33 @@ __device__ __forceinline__ void moduli_residues16(const double (&v)[16], int e, 
     double iv[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) iv[j] = rint(ldexp(v[j], P - e));
-    if (P <= 50) {
-        // |iv| <= 2^50: iv * (1/m) is within |iv| / m * 2^-52 < 1 / (2m) of
-        // iv / m, closer than iv / m ever lies to a half-integer it does
-        // not sit on, so q = rint(iv / m) exactly and r = iv - m q lies in
-        // [-m/2, m/2]; only m = 256 reaches +-128, and 128 wraps to -128,
-        // the same residue.
-        for (int l = 0; l < count; ++l) {
+    // |x| <= 2^50: x * (1/m) is within |x| / m * 2^-52 < 1 / (2m) of x / m,
+    // closer than x / m ever lies to a half-integer it does not sit on, so
+    // q = rint(x / m) exactly and r = x - m q lies in [-m/2, m/2]; only m = 256
+    // reaches +-128, and 128 wraps to -128, the same residue.
+    auto residues = [&](const double (&x)[16], int from, int to) {
+        for (int l = from; l < to; ++l) {
             const double m = (double)mods[l], im = inv_mods[l];
             union { i32x4 q; int8_t b[16]; } u;
 #pragma unroll
-            for (int j = 0; j < 16; ++j) u.b[j] = (int8_t)(int)fma(-m, rint(iv[j] * im), iv[j]);
+            for (int j = 0; j < 16; ++j) u.b[j] = (int8_t)(int)fma(-m, rint(x[j] * im), x[j]);
             store_residues16<BF16>(u.q, dst + (int64_t)l * plane);
         }
+    };
+    if (P <= 50) {
+        residues(iv, 0, count);
     } else {
-        for (int l = 0; l < count; ++l) {
-            const double m = (double)mods[l], im = inv_mods[l];
-            const int hi = (mods[l] - 1) / 2, lo = -(mods[l] / 2);
-            union { i32x4 q; int8_t b[16]; } u;
+        // Larger integers are first reduced modulo the product of the next
+        // MOD_GROUP moduli: the quotient is below 2^44 and within one of the
+        // true one, the FMA is exact, and the rest is below 2^48.  Three
+        // operations per value and group; a range correction per residue took
+        // six per value and modulus (3000 x 4100, 14 moduli, P = 51: 78 -> 58 us).
+        for (int l0 = 0; l0 < count; l0 += MOD_GROUP) {
+            const double M = kGroupProduct[l0 / MOD_GROUP], iM = kGroupInverse[l0 / MOD_GROUP];
+            double x[16];
 #pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                int r = (int)fma(-m, rint(iv[j] * im), iv[j]);   // exact: FMA of integers
-                if (r > hi) r -= mods[l];
-                if (r < lo) r += mods[l];
-                u.b[j] = (int8_t)r;
-            }
-            store_residues16<BF16>(u.q, dst + (int64_t)l * plane);
+            for (int j = 0; j < 16; ++j) x[j] = fma(-M, rint(iv[j] * iM), iv[j]);
+            residues(x, l0, l0 + MOD_GROUP < count ? l0 + MOD_GROUP : count);
         }
     }
 }
