@@ -7,7 +7,7 @@
 // them itself (src/cosma/local_multiply.cpp:341-349).
 //
 // Schedule.  C is cut into tile_m x tile_n tiles and k into tile_k panels
-// (the COSMA_GPU_MAX_TILE_{M,N,K} sizes of the handle).  Three kinds of work
+// (at most the COSMA_GPU_MAX_TILE_{M,N,K} sizes of the handle).  Three kinds of work
 // run on separate streams and are ordered only by events:
 //   * one host->device stream uploads operand blocks, in the order the tiles
 //     need them;
@@ -82,6 +82,7 @@ Kind classify(const void *p) {
 
 constexpr size_t SLOT_BYTES = 64ull << 20;   // pinned staging slot
 constexpr int N_SLOTS = 4;                   // per direction
+constexpr int64_t C_SLOTS = 4;               // device slots of incoming C tiles
 
 int grow(DevBuf &b, size_t bytes) {
     if (b.bytes >= bytes) return COSMA_AMD_OK;
@@ -314,6 +315,17 @@ static std::vector<std::pair<int64_t, int64_t>> shell_order(int64_t nTm, int64_t
     return out;
 }
 
+// Tile extent of the resident schedule where C's return counts (C at least an
+// eighth of A and B): up to four even tiles of about 1024 or more, within the
+// handle's tile size.  With two tiles, the first one of C is complete only when
+// most of A and B have arrived, and C's return trails the uploads (8192^3,
+// uploads 18.6 ms: 28.7 ms in 5000^3 tiles, 24.5 ms in 2048^3, 27.2 ms in 1024^3,
+// whose many strided block copies leave the link idle; 4096^3: 7.9 and 6.5 ms).
+static int64_t resident_tile(int64_t tile, int64_t extent) {
+    const int64_t parts = std::max<int64_t>(1, std::min<int64_t>(4, (extent + 256) / 1024));
+    return std::min(tile, ((extent + parts - 1) / parts + 127) / 128 * 128);
+}
+
 // Resident schedule: each block of A and B crosses the host link once, into a
 // device copy of the whole operand, and is reused by every tile that needs it.
 // The first floor(nTk/2) panels run panel-major over all tiles (the blocks of
@@ -323,8 +335,9 @@ static std::vector<std::pair<int64_t, int64_t>> shell_order(int64_t nTm, int64_t
 // the returns overlap the compute instead of trailing it.
 static int stream_resident(cosma_amd_handle_t h, const Operand &A, const Operand &B, Kind kc, int64_t m, int64_t n,
                            int64_t k, double alpha, double beta, double *c, int64_t ldc, bool copy_c_back,
-                           int64_t tm, int64_t tn, int64_t tk, int64_t nTm, int64_t nTn, int64_t nTk,
-                           bool defer_c, int64_t R) {
+                           int64_t tm, int64_t tn, int64_t tk, bool scale_only, bool defer_c) {
+    const int64_t nTm = (m + tm - 1) / tm, nTn = (n + tn - 1) / tn, nTk = scale_only ? 0 : (k + tk - 1) / tk;
+    const int64_t R = std::min<int64_t>(C_SLOTS, nTm * nTn);
     int rc;
     double *dA = const_cast<double *>(A.host), *dB = const_cast<double *>(B.host), *dC = c, *dC0 = nullptr;
     int64_t ldA = A.ld, ldB = B.ld, ldC = ldc;
@@ -593,7 +606,7 @@ static int stream_dgemm_body(cosma_amd_handle_t h, char ta, char tb, int64_t m, 
     // from a ring of R device slots, so that C uploads queue behind the
     // operand blocks that start the compute.
     const bool defer_c = kc != DEVICE && beta != 0.0 && nTk > 0;
-    const int64_t R = std::min<int64_t>(4, nTm * nTn);
+    const int64_t R = std::min<int64_t>(C_SLOTS, nTm * nTn);
 
     size_t free_b = 0, total_b = 0;
     CA_HIP(hipMemGetInfo(&free_b, &total_b));
@@ -613,8 +626,10 @@ static int stream_dgemm_body(cosma_amd_handle_t h, char ta, char tb, int64_t m, 
                   "(%zu bytes over a budget of %zu)", needA + needB + needC, limit);
         return COSMA_AMD_ERR_UNSUPPORTED;
     }
+    const bool finer = resident && !scale_only && kc != DEVICE && copy_c_back && 8 * (m * n) >= m * k + k * n;
     int rc = resident ? stream_resident(h, A, B, kc, m, n, k, alpha, beta, c, ldc, copy_c_back,
-                                        tm, tn, tk, nTm, nTn, nTk, defer_c, R)
+                                        finer ? resident_tile(tm, m) : tm, finer ? resident_tile(tn, n) : tn,
+                                        finer ? resident_tile(tk, k) : tk, scale_only, defer_c)
                       : stream_bounded(h, A, B, kc, m, n, k, alpha, beta, c, ldc,
                                        tm, tn, tk, nTm, nTn, nTk);
     if (rc) return rc;

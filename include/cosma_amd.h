@@ -194,7 +194,7 @@ int cosma_amd_dgemm_ozaki_noalloc(cosma_amd_handle_t handle, char transa, char t
  * pinned host memory (hipHostMalloc) or pageable host memory; the call
  * returns when C is final (on the host if copy_c_back != 0).
  * C is cut into tile_m x tile_n tiles and k into tile_k panels (the handle's
- * tile sizes, i.e. COSMA_GPU_MAX_TILE_{M,N,K}); uploads, per-tile MFMA DGEMMs
+ * tile sizes, i.e. COSMA_GPU_MAX_TILE_{M,N,K}, as upper bounds); uploads, per-tile MFMA DGEMMs
  * on the handle's round-robin streams (COSMA_GPU_STREAMS) and downloads of
  * finished C tiles overlap.  When A, B and C fit in the device-memory budget
  * (cosma_amd_handle_set_memory_limit, default 80% of free HBM) every block
