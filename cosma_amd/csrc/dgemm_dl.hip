@@ -4,16 +4,20 @@
 // any extents, leading dimensions and transposes.  The default kernel of
 // cosma_amd_dgemm.
 //
-//   * A workgroup of 2 x 2 waves owns a BM x BN tile of C, a wave a quarter of
-//     it in 16 x 16 MFMA blocks.  Five tile shapes, 128 x 128 to 32 x 32, all
+//   * A workgroup of 2 x 4 waves (2 x 2 below 64 x 64) owns a BM x BN tile of C,
+//     a wave its part in 16 x 16 MFMA blocks.  Five tile shapes, 128 x 128 to 32 x 32, all
 //     summing k in the order of dgemm.hip's gemm_tile: the choice of a tile
 //     (pick_dl_tile) never changes a bit of the result.
 //   * What bounds it: the FP64 MFMA pipe (a v_mfma_f64_16x16x4 takes 64
 //     cycles of a SIMD).  Two to four workgroups per CU share the pipe, so one's
-//     barrier and fragment reads overlap the others' MFMAs; NS LDS stages keep
-//     the loads of the next NS - 1 steps in flight, which is what a CU with a
-//     single workgroup needs (1024 x 1024 x 32768 TN, one 64 x 64 tile per CU:
-//     1332 us with two stages, 1000 us with three).
+//     barrier and fragment reads overlap the others' MFMAs, and eight waves of
+//     half the accumulators in place of four put twice the waves on a SIMD
+//     (128 x 128 tiles, two workgroups per CU: 8192^3 TN 72.3 -> 73.4 TF, NT 70.1 ->
+//     72.3; one workgroup per CU, 2048 x 2048 x 65536 TN: 69.4 -> 71.6; 64 x 64,
+//     1537 x 1021 x 2999 NT: 193 -> 177 us).  NS LDS stages keep the loads of the
+//     next NS - 1 steps in flight; small tiles need more than one (1024 x 1024 x
+//     32768 TN, one 64 x 64 tile per CU: 1332 us with two stages, 1000 us with
+//     three).
 //   * Fragment registers are double-buffered by half-step, and each batch of
 //     reads is waited for before the next one is issued (by then 8 to 32
 //     MFMAs old).  Left to the compiler, the wait stood behind the next batch
@@ -38,7 +42,6 @@ namespace cosma_amd {
 namespace {
 
 constexpr int BK = 16;       // k-step
-constexpr int NT = 256;      // threads per workgroup: 2 x 2 waves
 constexpr int NXCD = 8;
 
 typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));   // 16-byte access at 8-byte alignment
@@ -51,10 +54,12 @@ constexpr int WAIT_VM0_LGKM0 = 0x0070;
 // Slot (of eight) of k-pair kp in row r of a k-contiguous tile is kp ^ row_swz(r).
 __device__ __forceinline__ int row_swz(int r) { return ((r >> 2) & 3) | ((r & 2) << 1); }
 
-template <int R, bool KCONTIG>
+template <int R, bool KCONTIG, int NW>
 struct Operand {
+    static constexpr int NT = 64 * NW;
     static constexpr int SIZE = R * BK;          // doubles per stage
-    static constexpr int LOADS = R / 32;         // 1 KB wave instructions per wave and step
+    static constexpr int LOADS = R / 8 / NW;     // 1 KB wave instructions per wave and step
+    static_assert(R % (8 * NW) == 0 && NW % 4 == 0, "whole wave instructions, one k-pair parity per wave");
     static constexpr int NOFF = KCONTIG ? LOADS : 1;
     static constexpr int TAIL = R * BK / NT;     // elements per thread of the partial step
     const char *base;                            // wave-uniform
@@ -68,7 +73,7 @@ struct Operand {
             base = reinterpret_cast<const char *>(x + r0 * ld);
 #pragma unroll
             for (int q = 0; q < LOADS; ++q) {
-                const int row = 8 * (wave + 4 * q) + (lane >> 3);
+                const int row = 8 * (wave + NW * q) + (lane >> 3);
                 off[q] = (uint32_t)min(row, last) * (uint32_t)ldb + (uint32_t)(((lane & 7) ^ row_swz(row)) * 16);
             }
         } else {
@@ -85,10 +90,10 @@ struct Operand {
         for (int q = 0; q < LOADS; ++q) {
             // scalar base + 32-bit lane offset (the asm keeps the compiler from
             // folding the lane offset into 64-bit vector adds per load)
-            const char *u = KCONTIG ? base + (int64_t)k0 * 8 : base + (int64_t)(k0 + q * (512 / R)) * ldb;
+            const char *u = KCONTIG ? base + (int64_t)k0 * 8 : base + (int64_t)(k0 + q * (128 * NW / R)) * ldb;
             asm("" : "+s"(u));
             __builtin_amdgcn_global_load_lds(static_cast<const void *>(u + off[KCONTIG ? q : 0]),
-                                             (__attribute__((address_space(3))) void *)(tile + 128 * (wave + 4 * q)),
+                                             (__attribute__((address_space(3))) void *)(tile + 128 * (wave + NW * q)),
                                              16, 0, 0);
         }
     }
@@ -145,24 +150,24 @@ struct Frag {
 
 // One BM x BN tile of C at (m0, n0) with NS LDS stages in sm.  EDGE: the MFMAs
 // of 16 x 16 blocks that lie wholly outside C are skipped.
-template <int BM, int BN, int NS, bool AK, bool BKC, bool EDGE>
+template <int BM, int BN, int NS, int WM, int WN, bool AK, bool BKC, bool EDGE>
 __device__ __forceinline__ void dl_tile(int64_t M, int64_t N, int64_t K, double alpha, const double *__restrict__ A,
                                         int64_t lda, const double *__restrict__ B, int64_t ldb, double beta,
                                         double *__restrict__ C, int64_t ldc, int64_t m0, int64_t n0, double *sm) {
-    using OA = Operand<BM, AK>;
-    using OB = Operand<BN, BKC>;
+    using OA = Operand<BM, AK, WM * WN>;
+    using OB = Operand<BN, BKC, WM * WN>;
     constexpr int STAGE = OA::SIZE + OB::SIZE;
     constexpr int LOADS = OA::LOADS + OB::LOADS;
-    constexpr int FM = BM / 32, FN = BN / 32;
+    constexpr int FM = BM / 16 / WM, FN = BN / 16 / WN;
     constexpr bool EARLY_TAIL = BM * BN <= 64 * 64;
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave & 1, wn = wave >> 1;
+    const int wm = wave % WM, wn = wave / WM;
     const int g = lane >> 4, li = lane & 15;
     const OA oa(A, lda, m0, M, wave, lane);
     const OB ob(B, ldb, n0, N, wave, lane);
-    const Frag<BM, AK, FM> fra(wm * (BM / 2) + 4 * (li & 3) + (li >> 2), g);
-    const Frag<BN, BKC, FN> frb(wn * (BN / 2) + li, g);
+    const Frag<BM, AK, FM> fra(wm * (BM / WM) + 4 * (li & 3) + (li >> 2), g);
+    const Frag<BN, BKC, FN> frb(wn * (BN / WN) + li, g);
 
     // Full steps; a row-contiguous operand with an odd extent keeps the last
     // k out of them (the 16-byte load of its last row reads one element
@@ -188,8 +193,8 @@ __device__ __forceinline__ void dl_tile(int64_t M, int64_t N, int64_t K, double 
 #pragma unroll
         for (int j = 0; j < FN; ++j) bf[ks][j] = frb.read(tile + OA::SIZE, j, ks);
     };
-    const int rows_in = EDGE ? (int)min((int64_t)FM, (M - m0 - wm * (BM / 2) + 15) >> 4) : FM;   // may be <= 0
-    const int cols_in = EDGE ? (int)min((int64_t)FN, (N - n0 - wn * (BN / 2) + 15) >> 4) : FN;
+    const int rows_in = EDGE ? (int)min((int64_t)FM, (M - m0 - wm * (BM / WM) + 15) >> 4) : FM;   // may be <= 0
+    const int cols_in = EDGE ? (int)min((int64_t)FN, (N - n0 - wn * (BN / WN) + 15) >> 4) : FN;
     auto mfmas = [&](int h) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
@@ -264,10 +269,10 @@ __device__ __forceinline__ void dl_tile(int64_t M, int64_t N, int64_t K, double 
     const bool beta0 = (beta == 0.0);
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-        const int64_t row = m0 + wm * (BM / 2) + 16 * i + 4 * g;
+        const int64_t row = m0 + wm * (BM / WM) + 16 * i + 4 * g;
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-            const int64_t col = n0 + wn * (BN / 2) + 16 * j + li;
+            const int64_t col = n0 + wn * (BN / WN) + 16 * j + li;
             if (col >= N) continue;
             double *cp = C + row + col * ldc;
             const f64x4 r = acc[i][j];
@@ -296,9 +301,9 @@ __device__ __forceinline__ void dl_tile(int64_t M, int64_t N, int64_t K, double 
     }
 }
 
-// NS: LDS stages; WPE: waves per SIMD (= workgroups per CU) it is built for.
-template <int BM, int BN, int NS, int WPE, bool AK, bool BKC>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void dgemm_dl_kernel(
+// NS: LDS stages; WPE: waves per SIMD it is built for; WM x WN waves.
+template <int BM, int BN, int NS, int WPE, int WM, int WN, bool AK, bool BKC>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void dgemm_dl_kernel(
     int64_t M, int64_t N, int64_t K, double alpha,
     const double *__restrict__ A, int64_t lda,
     const double *__restrict__ B, int64_t ldb,
@@ -312,7 +317,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
     const uint32_t gsize = min((uint32_t)group_m, tiles_m - grp * group_m);
     const int64_t m0 = (int64_t)(grp * group_m + in_group % gsize) * BM;
     const int64_t n0 = (int64_t)(in_group / gsize) * BN;
-    dl_tile<BM, BN, NS, AK, BKC, false>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, m0, n0, sm);
+    dl_tile<BM, BN, NS, WM, WN, AK, BKC, false>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, m0, n0, sm);
 }
 
 // Grouped tiles: workgroup w takes the virtual ids w, w + G, ... of all
@@ -329,7 +334,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
 // balances its waves better at an edge, spilled and lost (774 us).
 constexpr int MIXED = 4;
 template <int BM, int BN, int NS, int WPE, int TRANS>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void dgemm_dl_grouped_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void dgemm_dl_grouped_kernel(
     const GroupedProblem *__restrict__ probs, const int *__restrict__ owner, int64_t total_tiles) {
     __shared__ __attribute__((aligned(16))) double sm[NS * (BM + BN) * BK];
     for (int64_t v = blockIdx.x; v < total_tiles; v += gridDim.x) {
@@ -342,7 +347,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
         const double alpha = scale_only ? 0.0 : q.alpha;
         if (v >= gridDim.x) __syncthreads();   // the previous tile's last LDS reads are done
 #define CA_TILE(X, Y)                                                                                           \
-    dl_tile<BM, BN, NS, X, Y, true>(q.m, q.n, K, alpha, q.a, q.lda, q.b, q.ldb, q.beta, q.c, q.ldc, m0, n0, sm)
+    dl_tile<BM, BN, NS, 2, 2, X, Y, true>(q.m, q.n, K, alpha, q.a, q.lda, q.b, q.ldb, q.beta, q.c, q.ldc, m0, n0, sm)
         switch (TRANS == MIXED ? q.flags & 3 : TRANS) {   // bit 0: A transposed, bit 1: B transposed
         case 0: CA_TILE(false, true); break;
         case 1: CA_TILE(true, true); break;
@@ -353,12 +358,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
     }
 }
 
-template <int BM, int BN, int NS, int WPE>
+template <int BM, int BN, int NS, int WPE, int WM, int WN>
 void launch(char ta, char tb, int64_t m, int64_t n, int64_t k, double alpha, const double *a, int64_t lda,
             const double *b, int64_t ldb, double beta, double *c, int64_t ldc, int group_m, hipStream_t s) {
-    const dim3 grid((unsigned)(((m + BM - 1) / BM) * ((n + BN - 1) / BN))), block(NT);
+    const dim3 grid((unsigned)(((m + BM - 1) / BM) * ((n + BN - 1) / BN))), block(64 * WM * WN);
 #define CA_LAUNCH_DL(X, Y)                                                                                        \
-    hipLaunchKernelGGL((dgemm_dl_kernel<BM, BN, NS, WPE, X, Y>), grid, block, 0, s, m, n, k, alpha, a, lda, b,   \
+    hipLaunchKernelGGL((dgemm_dl_kernel<BM, BN, NS, WPE, WM, WN, X, Y>), grid, block, 0, s, m, n, k, alpha, a, lda, b,   \
                        ldb, beta, c, ldc, group_m)
     // template flags: operand k-contiguous (A 'T', B 'N')
     if (ta == 'T' && tb == 'N') CA_LAUNCH_DL(true, true);
@@ -376,14 +381,17 @@ struct TileModel {
     int bm, bn;
     double extra;     // prologue and epilogue of a tile, in k
     double busy[3];   // MFMA utilisation with one, two, and more tiles per CU
+    double beyond;    // its factor when the operands exceed the last-level cache
 };
-// Fitted to 410 shapes (m, n 32 to 8192, k 8 to 32768, all transposes and
-// alignments, every tile timed): the choice is 0.6% slower than the fastest
-// tile on average, 14% at most.
+// Fitted to 420 shapes (m, n 32 to 8192, k 8 to 65536, all transposes and
+// alignments, every tile timed): the choice is 0.4% slower than the fastest
+// tile on average, 12% at most.
 constexpr TileModel MODEL[] = {
-    {128, 128, 210, {0.91, 0.913, 0.92}}, {64, 128, 98, {0.55, 0.66, 0.886}}, {64, 64, 62, {0.75, 0.785, 0.877}},
-    {64, 32, 60, {0.65, 0.70, 0.789}},    {32, 32, 56, {0.59, 0.654, 0.689}},
+    {128, 128, 97, {0.866, 0.924, 0.925}, 1.0}, {64, 128, 66, {0.689, 0.886, 0.912}, 0.977},
+    {64, 64, 66, {0.715, 0.804, 0.862}, 0.999}, {64, 32, 55, {0.623, 0.707, 0.774}, 0.784},
+    {32, 32, 52, {0.539, 0.622, 0.678}, 0.786},
 };
+constexpr double LLC_DOUBLES = 256.0 * (1 << 20) / 8;
 int64_t tiles_of(DlTile t, int64_t m, int64_t n) {
     return ((m + MODEL[t].bm - 1) / MODEL[t].bm) * ((n + MODEL[t].bn - 1) / MODEL[t].bn);
 }
@@ -392,15 +400,17 @@ int64_t tiles_of(DlTile t, int64_t m, int64_t n) {
 // The busiest CU computes ceil(tiles / CUs) tiles, each bm * bn * (k + extra)
 // products at the tile's MFMA utilisation: large tiles move less data per
 // product, small ones leave less of the chip idle and pad less.  1000^3 NN:
-// 132 us in 128 x 128 tiles (64 of 256 CUs busy), 38 us in 64 x 64; 1537 x
-// 1021 x 2999 NT: 381 us, 171 us in 32 x 32; 8192^3 NN: 15.2 ms, 18.6 ms.
+// 125 us in 128 x 128 tiles (64 of 256 CUs busy), 35 us in 64 x 64; 700 x 700 x
+// 16384 TN: 1914 us, 269 us in 64 x 32; 8192^3 TN: 14.8 ms, 18.6 ms in 32 x 32.
 DlTile pick_dl_tile(int64_t m, int64_t n, int64_t k) {
     DlTile best = DL_128x128;
     double least = 0.0;
+    const bool beyond = (double)(m + n) * (double)k > LLC_DOUBLES;
     for (int t = DL_128x128; t <= DL_32x32; ++t) {
         const TileModel &x = MODEL[t];
         const int64_t per_cu = (tiles_of(static_cast<DlTile>(t), m, n) + N_CU - 1) / N_CU;
-        const double cost = (double)(per_cu * x.bm * x.bn) * ((double)k + x.extra) / x.busy[std::min<int64_t>(per_cu, 3) - 1];
+        const double busy = x.busy[std::min<int64_t>(per_cu, 3) - 1] * (beyond ? x.beyond : 1.0);
+        const double cost = (double)(per_cu * x.bm * x.bn) * ((double)k + x.extra) / busy;
         if (t == DL_128x128 || cost < least) {
             least = cost;
             best = static_cast<DlTile>(t);
@@ -411,26 +421,21 @@ DlTile pick_dl_tile(int64_t m, int64_t n, int64_t k) {
 
 bool dl_fits(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb) {
     // 32-bit byte offsets over 128 rows, 32-bit step counts, and the 2^32
-    // work-items of a launch in the smallest tiles
-    return (m + 31) / 32 * ((n + 31) / 32) < ((int64_t)1 << 24) && k < ((int64_t)1 << 31) &&
+    // work-items of a launch
+    return (m + 31) / 32 * ((n + 31) / 32) < ((int64_t)1 << 23) && k < ((int64_t)1 << 31) &&
            lda < ((int64_t)1 << 22) && ldb < ((int64_t)1 << 22);
 }
 
 int launch_dl(DlTile tile, char ta, char tb, int64_t m, int64_t n, int64_t k, double alpha, const double *a, int64_t lda,
               const double *b, int64_t ldb, double beta, double *c, int64_t ldc, int group_m, hipStream_t s) {
-#define CA_DL(BM, BN, NS, WPE) \
-    launch<BM, BN, NS, WPE>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, group_m, s)
+#define CA_DL(BM, BN, NS, WPE, WM, WN) \
+    launch<BM, BN, NS, WPE, WM, WN>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, group_m, s)
     switch (tile) {
-    case DL_128x128: CA_DL(128, 128, 2, 2); break;
-    case DL_64x128: CA_DL(64, 128, 2, 3); break;
-    case DL_64x64: {
-        // one tile per CU and fewer: a third stage in place of the other workgroups
-        if (tiles_of(DL_64x64, m, n) <= N_CU) CA_DL(64, 64, 3, 3);
-        else CA_DL(64, 64, 2, 4);
-        break;
-    }
-    case DL_64x32: CA_DL(64, 32, 3, 4); break;
-    default: CA_DL(32, 32, 4, 4); break;
+    case DL_128x128: CA_DL(128, 128, 2, 4, 2, 4); break;
+    case DL_64x128: CA_DL(64, 128, 2, 6, 2, 4); break;
+    case DL_64x64: CA_DL(64, 64, 3, 6, 2, 4); break;
+    case DL_64x32: CA_DL(64, 32, 3, 4, 2, 2); break;
+    default: CA_DL(32, 32, 4, 4, 2, 2); break;
     }
 #undef CA_DL
     CA_HIP(hipGetLastError());
@@ -440,7 +445,7 @@ int launch_dl(DlTile tile, char ta, char tb, int64_t m, int64_t n, int64_t k, do
 int launch_grouped_dl(int cfg, const GroupedProblem *probs, int nprob, int64_t total_tiles, int grid, int trans,
                       hipStream_t s) {
     const int *owner = reinterpret_cast<const int *>(reinterpret_cast<const int64_t *>(probs + nprob) + nprob);
-    const dim3 g((unsigned)grid), b(NT);
+    const dim3 g((unsigned)grid), b(256);
 #define CA_GROUPED(BM, BN, NS, WPE, TRANS) \
     hipLaunchKernelGGL((dgemm_dl_grouped_kernel<BM, BN, NS, WPE, TRANS>), g, b, 0, s, probs, owner, total_tiles)
     switch (cfg) {

@@ -10,8 +10,8 @@ pytestmark = pytest.mark.gpu
 SHAPES = [
     (1, 1, 1), (1, 33, 16), (33, 1, 17), (31, 32, 15), (100, 97, 129), (33, 65, 1),   # 32 x 32
     (627, 2133, 101),                                                                  # 64 x 32
-    (1009, 1023, 2001), (1985, 2001, 333),                                             # 64 x 64, one / several per CU
-    (2417, 4007, 4001),                                                                # 64 x 128
+    (1009, 1023, 2001), (1283, 1391, 229), (2671, 967, 45),                            # 64 x 64, one to three per CU
+    (1985, 2001, 333), (2417, 4007, 4001),                                             # 64 x 128
     (3967, 3969, 3001),                                                                # 128 x 128
 ]
 
