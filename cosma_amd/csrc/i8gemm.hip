@@ -31,10 +31,9 @@ __device__ __forceinline__ auto mma(const i32x4 &a, const i32x4 &b, const std::c
         return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
 }
 
-// WIDE (EPI_RES8 with INT8 operands and K > 32768): the residue reduction
-// for sums of any magnitude (a template parameter so that each kernel holds
-// one form: both forms in one kernel made the register allocator spill).
-template <int EPI, bool BF16, bool WIDE = false>
+// EPI_RES8 with BF16 operands and EPI_F64ACC (i8gemm_dl_kernel takes the INT8
+// residue products).
+template <int EPI, bool BF16>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void i8gemm_kernel(I8Problem p, I8Jobs jobs) {
     using acc_t = std::conditional_t<BF16, f32x4, i32x4>;
     // LDS: two stages of 256 x 128-byte rows per operand (128 KB in all).
@@ -225,38 +224,30 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         // and each 16-byte chunk stays a contiguous chunk.
         // sym_mod's quarter-rate multiply and range corrections were most
         // of the epilogue's instructions.  sym_mod_odd_bits needs sums below
-        // 2^29 in magnitude, i.e. npairs * K <= 32768 (|x| <= npairs * K *
-        // 2^14; the BF16 sums stay below 2^24 for every K), else
-        // sym_mod_odd_bits_wide applies.
-        // Both return a word whose low byte is x's residue also for m = 256
+        // 2^29 in magnitude (the BF16 sums stay below 2^24 for every K) and
+        // returns a word whose low byte is x's residue also for m = 256
         // (c16 = 0: y = x & 0xffff, and y - q m = x mod 256 whatever q);
         // even moduli other than 256 are rejected at launch.
         uint8_t *tile = reinterpret_cast<uint8_t *>(&sa[0][0]);
         __syncthreads();
-        auto stage = [&](auto residue_bits) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int rt = wm * 128 + 16 * i + 4 * g;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int ct = wn * 128 + 16 * j + li;
-                    uint32_t b[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) b[e] = residue_bits((int)acc[i][j][e]);   // BF16: exact integers
-                    // low bytes of b[0..3] -> one word (v_perm_b32 picks bytes 0-3 of its
-                    // second operand and 4-7 of its first; selector 0x0c gives zero)
-                    const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u);
-                    const uint32_t hi = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u);
-                    *reinterpret_cast<uint32_t *>(tile + ct * 256 + (rt ^ (16 * (ct & 15)))) =
-                        __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-                }
-            }
-        };
         const float c16 = jobs.fmod[z][2];
-        if constexpr (WIDE)
-            stage([&](int x) { return sym_mod_odd_bits_wide(x, c16, finv_m, neg_m); });
-        else
-            stage([&](int x) { return sym_mod_odd_bits(x, c16, finv_m, neg_m); });
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int rt = wm * 128 + 16 * i + 4 * g;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int ct = wn * 128 + 16 * j + li;
+                uint32_t b[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) b[e] = sym_mod_odd_bits((int)acc[i][j][e], c16, finv_m, neg_m);   // exact integers
+                // low bytes of b[0..3] -> one word (v_perm_b32 picks bytes 0-3 of its
+                // second operand and 4-7 of its first; selector 0x0c gives zero)
+                const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u);
+                const uint32_t hi = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u);
+                *reinterpret_cast<uint32_t *>(tile + ct * 256 + (rt ^ (16 * (ct & 15)))) =
+                    __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+            }
+        }
         __syncthreads();
         int8_t *out = static_cast<int8_t *>(p.out) + (int64_t)z * p.out_stride;
 #pragma unroll
@@ -290,6 +281,159 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void
                     o[e] = p.accumulate ? o[e] + val : val;
                 }
             }
+        }
+    }
+}
+
+// The INT8 residue products on eight waves (2 x 4, 128 x 64 of the tile each):
+// two waves per SIMD, so that one's barrier and fragment reads run under the
+// other's MFMAs, and operand tiles straight from global memory into LDS
+// (global_load_lds_dwordx4), which leaves the registers to the accumulators
+// (128) and two half-steps of fragments (96).  Rows of 128 bytes in LDS with
+// chunk c of row r at c ^ (r & 7); the loads' global addresses apply it.
+// WIDE (K > 32768): the residue reduction for sums of any magnitude.
+// What bounds it: power first, then LDS.  14 products of 8192^3 take 6.23 ms
+// (2.47 POPS; 6.38 ms on four waves of 128 x 128 with register-staged loads) on
+// random operands, 5.52 ms (5.80 ms) where all residues of a plane are equal
+// and the clock holds, 4.87 ms with all loads hitting L2 as well; the step's 260
+// KB through LDS alone take 2030 of the 2048 cycles of its MFMAs.
+typedef __attribute__((address_space(3))) void lds_void;
+constexpr int NT8 = 512;
+constexpr int wait_vm(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0F70; }
+constexpr int WAIT_LGKM0 = 0xC07F;
+template <bool WIDE>
+__global__ __launch_bounds__(NT8) __attribute__((amdgpu_waves_per_eu(2, 2))) void i8gemm_dl_kernel(I8Problem p, I8Jobs jobs) {
+    __shared__ __attribute__((aligned(16))) int8_t sm[2][(BM + BN) * BK];   // 128 KB
+    const int z = blockIdx.y;
+    const uint32_t tiles_m = (uint32_t)((p.M + BM - 1) / BM), tiles_n = (uint32_t)((p.N + BN - 1) / BN);
+    const uint32_t bid = (uint32_t)xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t per_group = GROUP_M * tiles_n, grp = bid / per_group, in_group = bid - grp * per_group;
+    const uint32_t gsize = min((uint32_t)GROUP_M, tiles_m - grp * GROUP_M);
+    const int64_t m0 = (int64_t)(grp * GROUP_M + in_group % gsize) * BM;
+    const int64_t n0 = (int64_t)(in_group / gsize) * BN;
+
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    const int g = lane >> 4, li = lane & 15;
+    constexpr int FM = 8, FN = 4, LOADS = 8;
+
+    const int ksteps = (int)(p.K / BK), nsteps = jobs.npairs[z] * ksteps, last = nsteps - 1;
+    uint64_t pa_bits = 0, pb_bits = 0;
+#pragma unroll
+    for (int q = 0; q < I8_MAX_PAIRS; ++q) {
+        pa_bits |= (uint64_t)jobs.pa[z][q] << (8 * q);
+        pb_bits |= (uint64_t)jobs.pb[z][q] << (8 * q);
+    }
+    // wave instruction q of a step: rows 8 (wave + 8 q) .. + 7
+    const int lrow = 8 * wave + (lane >> 3), chunk = (lane & 7) ^ (lane >> 3);
+    const uint32_t offa = (uint32_t)lrow * (uint32_t)p.lda + 16u * chunk;
+    const uint32_t offb = (uint32_t)lrow * (uint32_t)p.ldb + 16u * chunk;
+    auto issue = [&](int step, int st) {
+        const int pair = step / ksteps;
+        const int64_t k0 = (int64_t)(step - pair * ksteps) * BK;
+        const int8_t *A = p.a + (int64_t)((pa_bits >> (8 * pair)) & 0xff) * p.a_stride + m0 * p.lda + k0;
+        const int8_t *B = p.b + (int64_t)((pb_bits >> (8 * pair)) & 0xff) * p.b_stride + n0 * p.ldb + k0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int8_t *ua = A + q * 64 * p.lda, *ub = B + q * 64 * p.ldb;
+            asm("" : "+s"(ua), "+s"(ub));
+            __builtin_amdgcn_global_load_lds(static_cast<const void *>(ua + offa), (lds_void *)(sm[st] + 1024 * (wave + 8 * q)), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(static_cast<const void *>(ub + offb), (lds_void *)(sm[st] + BM * BK + 1024 * (wave + 8 * q)), 16, 0, 0);
+        }
+    };
+    i32x4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = i32x4{0, 0, 0, 0};
+    i32x4 fa[2][FM], fb[2][FN];
+    const int ra0 = (wm * 128 + li) * BK, rb0 = BM * BK + (wn * 64 + li) * BK;
+    const int c0 = 16 * (g ^ (li & 7)), c1 = 16 * ((g + 4) ^ (li & 7));
+    auto read_frags = [&](int st, int h) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) fb[h][j] = *reinterpret_cast<const i32x4 *>(sm[st] + rb0 + 16 * BK * j + (h ? c1 : c0));
+#pragma unroll
+        for (int i = 0; i < FM; ++i) fa[h][i] = *reinterpret_cast<const i32x4 *>(sm[st] + ra0 + 16 * BK * i + (h ? c1 : c0));
+    };
+    auto mfmas = [&](int h) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[h][i], fb[h][j], acc[i][j], 0, 0, 0);
+    };
+    auto barrier = [&]() {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    // The schedule of the FP64 direct-LDS kernel: half-step 1 is read under the
+    // MFMAs of half-step 0, half-step 0 of the next step under those of 1, each
+    // batch of reads waited for before the next; the loads have a whole step.
+    auto iteration = [&](int s, int st) {
+        __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);
+        __builtin_amdgcn_sched_barrier(0);
+        read_frags(st, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        mfmas(0);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(wait_vm(0) & WAIT_LGKM0);
+        barrier();
+        issue(min(s + 2, last), st);
+        __builtin_amdgcn_sched_barrier(0);
+        read_frags(st ^ 1, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        mfmas(1);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (nsteps > 0) {
+        issue(0, 0);
+        issue(min(1, last), 1);
+        __builtin_amdgcn_s_waitcnt(wait_vm(LOADS));
+        barrier();
+        read_frags(0, 0);
+        for (int s = 0; s < nsteps; s += 2) {   // nsteps is even
+            iteration(s, 0);
+            iteration(s + 1, 1);
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(wait_vm(0) & WAIT_LGKM0);   // no LDS writes outstanding
+    barrier();
+
+    // ---- epilogue: i8gemm_kernel's
+    const float finv_m = jobs.fmod[z][0], neg_m = jobs.fmod[z][1], c16 = jobs.fmod[z][2];
+    uint8_t *tile = reinterpret_cast<uint8_t *>(&sm[0][0]);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+        const int rt = wm * 128 + 16 * i + 4 * g;
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            const int ct = wn * 64 + 16 * j + li;
+            uint32_t b[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                b[e] = WIDE ? sym_mod_odd_bits_wide(acc[i][j][e], c16, finv_m, neg_m)
+                            : sym_mod_odd_bits(acc[i][j][e], c16, finv_m, neg_m);
+            const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u);
+            const uint32_t hi = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u);
+            *reinterpret_cast<uint32_t *>(tile + ct * 256 + (rt ^ (16 * (ct & 15)))) =
+                __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+        }
+    }
+    __syncthreads();
+    int8_t *out = static_cast<int8_t *>(p.out) + (int64_t)z * p.out_stride;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const int id = t + NT8 * q, ct = id >> 4, c = id & 15;
+        const int64_t col = n0 + ct, row = m0 + 16 * c;
+        if (col >= p.N || row >= p.M) continue;
+        const i32x4 v = *reinterpret_cast<const i32x4 *>(tile + ct * 256 + 16 * (c ^ (ct & 15)));
+        int8_t *o = out + row + col * p.ldo;
+        if (row + 16 <= p.M) {
+            *reinterpret_cast<i32x4 *>(o) = v;
+        } else {
+            union { i32x4 q; int8_t b[16]; } u;
+            u.q = v;
+            for (int e = 0; e < 16 && row + e < p.M; ++e) o[e] = u.b[e];
         }
     }
 }
@@ -344,8 +488,8 @@ int launch_i8gemm(const I8Problem &p, const I8Jobs &jobs, int Z, I8Epilogue epi,
     switch (epi) {
     case EPI_RES8:
         if (p.bf16) hipLaunchKernelGGL((i8gemm_kernel<EPI_RES8, true>), grid, block, 0, s, p, j);
-        else if (sum_len <= 32768) hipLaunchKernelGGL((i8gemm_kernel<EPI_RES8, false>), grid, block, 0, s, p, j);
-        else hipLaunchKernelGGL((i8gemm_kernel<EPI_RES8, false, true>), grid, block, 0, s, p, j);
+        else if (sum_len <= 32768) hipLaunchKernelGGL(i8gemm_dl_kernel<false>, grid, dim3(NT8), 0, s, p, j);
+        else hipLaunchKernelGGL(i8gemm_dl_kernel<true>, grid, dim3(NT8), 0, s, p, j);
         break;
     default: hipLaunchKernelGGL((i8gemm_kernel<EPI_F64ACC, false>), grid, block, 0, s, p, j); break;
     }

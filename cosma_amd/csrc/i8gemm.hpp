@@ -16,6 +16,8 @@
 //   EPI_F64ACC  C64 = scale * acc (+ C64 if accumulate) in FP64 (slices method;
 //               jobs of one launch must write disjoint outputs).
 //
+// INT8 residue products (EPI_RES8): 256 x 256 tiles on eight waves, see
+// i8gemm_dl_kernel.  The others:
 // Tile: 256 x 256 per workgroup of 256 threads (2 x 2 waves of 128 x 128, i.e.
 // 8 x 8 MFMA blocks of 16 x 16 per wave, 256 INT32 accumulators per lane in
 // AGPRs), k-step 128 (two MFMA depths: every row of a global load is one
