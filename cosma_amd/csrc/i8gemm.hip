@@ -31,8 +31,8 @@ __device__ __forceinline__ auto mma(const i32x4 &a, const i32x4 &b, const std::c
         return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
 }
 
-// EPI_RES8 with BF16 operands and EPI_F64ACC (i8gemm_dl_kernel takes the INT8
-// residue products).
+// EPI_RES8 with BF16 operands or very large INT8 planes and EPI_F64ACC
+// (i8gemm_dl_kernel takes the other INT8 residue products).
 template <int EPI, bool BF16>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void i8gemm_kernel(I8Problem p, I8Jobs jobs) {
     using acc_t = std::conditional_t<BF16, f32x4, i32x4>;
@@ -224,7 +224,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         // and each 16-byte chunk stays a contiguous chunk.
         // sym_mod's quarter-rate multiply and range corrections were most
         // of the epilogue's instructions.  sym_mod_odd_bits needs sums below
-        // 2^29 in magnitude (the BF16 sums stay below 2^24 for every K) and
+        // 2^29 in magnitude, i.e. npairs * K <= 32768 (|x| <= npairs * K *
+        // 2^14; the BF16 sums stay below 2^24 for every K), and
         // returns a word whose low byte is x's residue also for m = 256
         // (c16 = 0: y = x & 0xffff, and y - q m = x mod 256 whatever q);
         // even moduli other than 256 are rejected at launch.
@@ -488,8 +489,12 @@ int launch_i8gemm(const I8Problem &p, const I8Jobs &jobs, int Z, I8Epilogue epi,
     switch (epi) {
     case EPI_RES8:
         if (p.bf16) hipLaunchKernelGGL((i8gemm_kernel<EPI_RES8, true>), grid, block, 0, s, p, j);
-        else if (sum_len <= 32768) hipLaunchKernelGGL(i8gemm_dl_kernel<false>, grid, dim3(NT8), 0, s, p, j);
-        else hipLaunchKernelGGL(i8gemm_dl_kernel<true>, grid, dim3(NT8), 0, s, p, j);
+        else if (sum_len > 32768) hipLaunchKernelGGL(i8gemm_dl_kernel<true>, grid, dim3(NT8), 0, s, p, j);
+        // Operand planes well beyond the 256 MB last-level cache: the four-wave
+        // kernel's loads have two steps to land (registers, then LDS), the other's
+        // one (16384^3, 14 products: 47.9 and 49.2 ms; 12288^3: 21.4 and 21.0 ms).
+        else if ((p.M + p.N) * p.K > ((int64_t)384 << 20)) hipLaunchKernelGGL((i8gemm_kernel<EPI_RES8, false>), grid, block, 0, s, p, j);
+        else hipLaunchKernelGGL(i8gemm_dl_kernel<false>, grid, dim3(NT8), 0, s, p, j);
         break;
     default: hipLaunchKernelGGL((i8gemm_kernel<EPI_F64ACC, false>), grid, block, 0, s, p, j); break;
     }
