@@ -23,7 +23,10 @@
 //     MFMAs old).  Left to the compiler, the wait stood behind the next batch
 //     and covered it too, idling the wave for an LDS round trip per half-step
 //     (8192^3 TN 70.6 -> 73.0 TF, NN 70.7 -> 72.1 with the scalar addresses).
-//   * LDS layout per operand and stage, both free of bank conflicts:
+//   * LDS layout per operand and stage, every eight lanes of a fragment read on
+//     distinct 16-byte bank groups (SQ_LDS_BANK_CONFLICT still counts 1.3
+//     cycles per LDS instruction at 16384^3 TN, in total what the former slot
+//     function kp ^ (r & 7), two-way by that measure, counted):
 //     k-contiguous (A 'T', B 'N'): row r holds its eight k-pairs in 128 bytes,
 //     pair kp in slot kp ^ row_swz(r); a fragment is one 16-byte read.
 //     Row-contiguous (A 'N', B 'T'): k-row k holds the tile's rows, row r at
