@@ -106,6 +106,7 @@ __global__ __launch_bounds__(NT) void copy_kernel(int64_t rows, int64_t cols, do
 // or keep alive.
 constexpr int LIST = 72;     // blocks per launch (3.5 KB of the 4 KB of arguments)
 constexpr int ITEMS = 8;     // pairs per thread
+constexpr int64_t LIST_PAIRS = 1 << 26;   // most pairs of one block
 struct BlockList {
     struct {
         const double *src;
@@ -356,8 +357,9 @@ int launch_block_transform(char op, int64_t rows, int64_t cols, double alpha,
     // 5001: 111 and 79 us, but 3000 x 5000: 46 and 53 us)
     const bool large = rows * cols >= 20000000;
     if (op == 'N') {
-        // a 512-row window would leave most threads idle (40 x 100000: 25 -> 15 us)
-        if (rows <= NT && rows * cols >= (1 << 20) && rows * cols <= (1 << 26)) {
+        // a 512-row window would leave most threads idle (40 x 100000: 25 -> 15 us;
+        // 1 x 10^8: 9.2 -> 2.4 ms, 240 x 2000000: 1.91 -> 1.53 ms)
+        if (rows <= NT && rows * cols >= (1 << 20)) {
             const CopyBlock one{src, dst, lds, ldd, rows, cols};
             return launch_block_copies(&one, 1, alpha, beta, s);
         }
@@ -423,15 +425,22 @@ int launch_block_copies(const CopyBlock *blocks, int64_t n, double alpha, double
     for (int64_t i = 0; i < n; ++i) {
         const CopyBlock &b = blocks[i];
         if (b.rows == 0 || b.cols == 0) continue;
-        const int64_t pairs = (b.rows + LINE) / 2, total = pairs * b.cols;
-        if (b.rows > (1 << 26) || b.cols > (1 << 26) || total > (1 << 26)) {   // 1 GiB fills the chip by itself
+        const int64_t pairs = (b.rows + LINE) / 2;
+        if (b.rows > NT && pairs * b.cols > LIST_PAIRS) {   // 1 GiB fills the chip by itself
             rc = launch_block_transform('N', b.rows, b.cols, alpha, b.src, b.lds, beta, b.dst, b.ldd, s);
             if (rc) return rc;
             continue;
         }
-        list.b[list.n++] = {b.src, b.dst, b.lds, b.ldd, (int)b.rows, (int)b.cols, groups, (uint32_t)pairs};
-        groups += (uint32_t)((total + NT * ITEMS - 1) / (NT * ITEMS));
-        if (list.n == LIST && (rc = flush())) return rc;
+        // Narrow blocks stay here whatever their length (launch_block_transform
+        // sends them to this list), cut to the kernel's 32-bit indexes.
+        const int64_t piece = b.rows > NT ? b.cols : LIST_PAIRS / pairs;
+        for (int64_t c0 = 0; c0 < b.cols; c0 += piece) {
+            const int64_t nc = std::min(piece, b.cols - c0);
+            list.b[list.n++] = {b.src + c0 * b.lds, b.dst + c0 * b.ldd, b.lds, b.ldd, (int)b.rows, (int)nc, groups,
+                                (uint32_t)pairs};
+            groups += (uint32_t)((pairs * nc + NT * ITEMS - 1) / (NT * ITEMS));
+            if (list.n == LIST && (rc = flush())) return rc;
+        }
     }
     return flush();
 }

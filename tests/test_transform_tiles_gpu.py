@@ -24,6 +24,7 @@ def matrix(rows, cols, pad, offset, seed):
     ("N", 1, 1, 0, 0, 0, 0), ("N", 1023, 70, 1, 0, 1, 0), ("N", 1025, 65, 0, 3, 0, 1),   # cached, without and with shift
     ("N", 4099, 4097, 0, 2, 1, 1), ("N", 4096, 4096, 0, 0, 0, 0),                        # streamed
     ("N", 1, 1048577, 0, 1, 0, 1), ("N", 255, 4200, 2, 0, 0, 1), ("N", 256, 4096, 0, 0, 0, 0),   # narrow
+    ("N", 1, (1 << 23) + 1, 0, 1, 0, 0), ("N", 3, (1 << 24) - 1, 1, 0, 1, 1),             # narrow, cut in pieces
     ("T", 1024, 19532, 1, 0, 0, 1), ("T", 5001, 4003, 0, 1, 1, 0), ("T", 19532, 1024, 0, 0, 0, 0),   # shifted
     ("T", 4096, 16384, 0, 0, 0, 0), ("T", 4111, 16401, 15, 1, 0, 0),                    # whole lines
 ])
