@@ -626,10 +626,20 @@ static int stream_dgemm_body(cosma_amd_handle_t h, char ta, char tb, int64_t m, 
                   "(%zu bytes over a budget of %zu)", needA + needB + needC, limit);
         return COSMA_AMD_ERR_UNSUPPORTED;
     }
-    const bool finer = resident && !scale_only && kc != DEVICE && copy_c_back && 8 * (m * n) >= m * k + k * n;
+    int64_t fm = tm, fn = tn, fk = tk;
+    if (resident && !scale_only && kc != DEVICE && copy_c_back && 8 * (m * n) >= m * k + k * n) {
+        // Four slots of tiles rounded up to 128 can hold more than one coarse
+        // tile's slot (1793 x 1793: 34 MB and 26 MB): only within the budget.
+        const int64_t rm = resident_tile(tm, m), rn = resident_tile(tn, n);
+        const int64_t slots = std::min<int64_t>(C_SLOTS, ((m + rm - 1) / rm) * ((n + rn - 1) / rn));
+        if (!defer_c || needA + needB + needC + (size_t)slots * rm * rn * 8 <= limit) {
+            fm = rm;
+            fn = rn;
+            fk = resident_tile(tk, k);
+        }
+    }
     int rc = resident ? stream_resident(h, A, B, kc, m, n, k, alpha, beta, c, ldc, copy_c_back,
-                                        finer ? resident_tile(tm, m) : tm, finer ? resident_tile(tn, n) : tn,
-                                        finer ? resident_tile(tk, k) : tk, scale_only, defer_c)
+                                        fm, fn, fk, scale_only, defer_c)
                       : stream_bounded(h, A, B, kc, m, n, k, alpha, beta, c, ldc,
                                        tm, tn, tk, nTm, nTn, nTk);
     if (rc) return rc;

@@ -38,3 +38,30 @@ def test_default_tiles(handle, ta, tb, m, n, k, beta, pin):
     diff = (hC - want)[:, :m].norm() / want[:, :m].norm()
     assert diff <= 2 * gemm_bound(k)
     assert torch.equal(hC[:, m], want[:, m])
+
+
+def test_finer_tiles_keep_to_the_memory_limit():
+    """The limit admits one slot of the whole C, not the four of 1024 x 1024 that need 8 MB more: those are
+    allocated (here: refused) only once the limit is lifted."""
+    import torch
+    import cosma_amd as ca
+    m, n, k = 1793, 1793, 64
+    h = ca.Handle(0)
+    A, B, C = (torch.rand(s, dtype=torch.float64).pin_memory() for s in ((k, m), (n, k), (n, m)))
+    want = 1.5 * (B @ A) + 0.5 * C
+
+    def product():
+        h.dgemm_host("N", "N", m, n, k, 1.5, A.data_ptr(), m, B.data_ptr(), k, 0.5, C.data_ptr(), m)
+        assert h.last_mode() == 1
+
+    h.set_memory_limit(8 * (m * k + k * n + 2 * m * n))
+    product()
+    assert (C - want).norm() / want.norm() <= 2 * gemm_bound(k)
+    h.set_memory_limit(0)
+    ca.fail_allocations(0, 1)
+    try:
+        with pytest.raises(ca.CosmaAmdError) as e:
+            product()
+        assert e.value.status == 3
+    finally:
+        ca.fail_allocations(0, 0)
