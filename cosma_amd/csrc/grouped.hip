@@ -160,10 +160,10 @@ int grouped_create(cosma_amd_handle_t h, const cosma_amd_gemm_desc *d, int64_t c
         // descriptors, then their first tile indices (the kernels' search array)
         std::vector<int64_t> starts;
         for (const GroupedProblem &g : sorted) starts.push_back(g.tile_start);
-        // and the owner of every tile
+        // and the owner of every tile (direct-LDS kernels)
         std::vector<int> owner;
-        owner.reserve((size_t)t);
-        for (size_t i = 0; i < sorted.size(); ++i)
+        if (p->dl >= 0) owner.reserve((size_t)t);
+        for (size_t i = 0; p->dl >= 0 && i < sorted.size(); ++i)
             owner.insert(owner.end(), (size_t)((i + 1 < sorted.size() ? starts[i + 1] : t) - starts[i]), (int)i);
         const size_t dbytes = sorted.size() * sizeof(GroupedProblem), sbytes = starts.size() * sizeof(int64_t);
         const size_t obytes = owner.size() * sizeof(int);
@@ -177,7 +177,7 @@ int grouped_create(cosma_amd_handle_t h, const cosma_amd_gemm_desc *d, int64_t c
         e = hipMemcpy(p->dev[cfg], sorted.data(), dbytes, hipMemcpyHostToDevice);
         if (e == hipSuccess)
             e = hipMemcpy(reinterpret_cast<char *>(p->dev[cfg]) + dbytes, starts.data(), sbytes, hipMemcpyHostToDevice);
-        if (e == hipSuccess)
+        if (e == hipSuccess && obytes > 0)
             e = hipMemcpy(reinterpret_cast<char *>(p->dev[cfg]) + dbytes + sbytes, owner.data(), obytes, hipMemcpyHostToDevice);
         if (e != hipSuccess) {
             set_error("grouped dgemm: descriptor upload failed (%s)", hipGetErrorString(e));
