@@ -6,6 +6,10 @@
 // (src/cosma/local_multiply.cpp:299-381 -> Tiled-MM gpu::gemm at :245-260,
 // or cosma::gemm -> cblas_dgemm at src/cosma/blas.cpp:24-48).
 //
+// The entry points use the direct-LDS kernels (dgemm_dl.hip) wherever their
+// 32-bit offsets reach; this file's kernels, staged through registers, take
+// the rest and the explicit tile configurations.
+//
 // Work decomposition
 //   * A 256-thread workgroup (4 waves of 64 lanes, 2 x 2) owns a BM x BN block
 //     of C; each wave owns a (BM/2) x (BN/2) quarter made of FM x FN MFMA
