@@ -273,26 +273,42 @@ __global__ __launch_bounds__(NT) void transpose_cached_vec_kernel(int64_t rows, 
 
 // dst(rows x cols)[i, j] <- f(src[j, i]); src is cols x rows with leading dim
 // lds.  Tiles of TR dst rows x TC dst columns, SHIFT: each column's rows start
-// at its own line boundary at or up to 15 rows after the tile's first.
-template <int TR, int TC, bool SHIFT>
+// at its own line boundary at or up to 15 rows after the tile's first.  BETA:
+// dst is read (mode 2), by loads in flight together with those of src.
+template <int TR, int TC, bool SHIFT, bool BETA>
 __global__ __launch_bounds__(NT) void transpose_kernel(int64_t rows, int64_t cols, double alpha,
                                                        const double *__restrict__ src, int64_t lds,
                                                        double beta, double *__restrict__ dst,
                                                        int64_t ldd, int mode, uint32_t nx, uint32_t tiles) {
     constexpr int S = SHIFT ? LINE : 0, LR = TR + S, H = TC / 2;
-    static_assert(TR % LINE == 0 && LR * H % NT == 0 && TR * TC % (2 * NT) == 0, "whole rounds of the workgroup");
+    static_assert(TR % LINE == 0 && LR * H % NT == 0 && TR * TC % (2 * NT) == 0 && LR * TC % NT == 0, "whole rounds of the workgroup");
     __shared__ double tile[LR][TC + 1];
     const int t = threadIdx.x;
     for (uint32_t b = blockIdx.x; b < tiles; b += gridDim.x) {
         const int64_t i0 = (int64_t)(b % nx) * TR - S, j0 = (int64_t)(b / nx) * TC;
         auto shift = [&](const double *col) { return SHIFT ? (LINE - phase(col)) & (LINE - 1) : 0; };
         if (i0 >= 0 && i0 + LR <= rows && j0 + TC <= cols) {
-            f64x2u v[LR * H / NT];
+            constexpr int OUT = TR * TC / 2 / NT;
+            f64x2u v[LR * H / NT], old[OUT];
+            auto dst_pair = [&](int q, int &jl, int &r) {
+                const int e = t + NT * q;
+                jl = e / (TR / 2);
+                double *col = dst + (j0 + jl) * ldd + i0;
+                r = (e % (TR / 2)) * 2 + shift(col);
+                return reinterpret_cast<f64x2u *>(col + r);
+            };
 #pragma unroll
             for (int q = 0; q < LR * H / NT; ++q) {
                 const int e = t + NT * q, il = e / H, c2 = (e % H) * 2;
                 const f64x2u *p = reinterpret_cast<const f64x2u *>(src + (j0 + c2) + (i0 + il) * lds);
                 v[q] = SHIFT ? *p : __builtin_nontemporal_load(p);
+            }
+            if (BETA) {
+#pragma unroll
+                for (int q = 0; q < OUT; ++q) {
+                    int jl, r;
+                    old[q] = *dst_pair(q, jl, r);
+                }
             }
 #pragma unroll
             for (int q = 0; q < LR * H / NT; ++q) {
@@ -302,28 +318,41 @@ __global__ __launch_bounds__(NT) void transpose_kernel(int64_t rows, int64_t col
             }
             __syncthreads();
 #pragma unroll
-            for (int q = 0; q < TR * TC / 2 / NT; ++q) {
-                const int e = t + NT * q, jl = e / (TR / 2);
-                double *col = dst + (j0 + jl) * ldd + i0;
-                const int r = (e % (TR / 2)) * 2 + shift(col);
-                f64x2u *d = reinterpret_cast<f64x2u *>(col + r);
-                const f64x2u old = mode == 2 ? *d : f64x2u{0.0, 0.0};
-                __builtin_nontemporal_store(combine2(f64x2u{tile[r][jl], tile[r + 1][jl]}, alpha, beta, old, mode), d);
+            for (int q = 0; q < OUT; ++q) {
+                int jl, r;
+                f64x2u *d = dst_pair(q, jl, r);
+                __builtin_nontemporal_store(combine2(f64x2u{tile[r][jl], tile[r + 1][jl]}, alpha, beta, old[q], BETA ? 2 : mode), d);
             }
         } else {
-            for (int e = t; e < LR * TC; e += NT) {
-                const int il = e / TC, c = e % TC;
-                const int64_t i = i0 + il, j = j0 + c;
-                if (i >= 0 && i < rows && j < cols) tile[il][c] = src[j + i * lds];
+            // Edge tile: by element, from addresses clamped into the matrix so
+            // that no load waits for another (one element at a time, two edge
+            // tiles in 24 made 2601 x 12501 take 308 us with beta = 1/2).
+            constexpr int IN = LR * TC / NT, OUT = TR * TC / NT;
+            double v[IN], old[OUT];
+#pragma unroll
+            for (int q = 0; q < IN; ++q) {
+                const int e = t + NT * q;
+                const int64_t i = min(max(i0 + e / TC, (int64_t)0), rows - 1), j = min(j0 + e % TC, cols - 1);
+                v[q] = src[j + i * lds];
             }
+            if (BETA) {
+#pragma unroll
+                for (int q = 0; q < OUT; ++q) {
+                    const int e = t + NT * q;
+                    double *col = dst + min(j0 + e / TR, cols - 1) * ldd;
+                    old[q] = col[min(max(i0 + e % TR + shift(col + i0), (int64_t)0), rows - 1)];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < IN; ++q) tile[(t + NT * q) / TC][(t + NT * q) % TC] = v[q];
             __syncthreads();
-            for (int e = t; e < TR * TC; e += NT) {
-                const int jl = e / TR;
-                const int64_t j = j0 + jl;
-                if (j >= cols) break;
-                double *col = dst + j * ldd + i0;
+#pragma unroll
+            for (int q = 0; q < OUT; ++q) {
+                const int e = t + NT * q, jl = e / TR;
+                double *col = dst + (j0 + jl) * ldd + i0;
                 const int r = e % TR + shift(col);
-                if (i0 + r >= 0 && i0 + r < rows) col[r] = combine(tile[r][jl], alpha, beta, col + r, mode);
+                if (j0 + jl < cols && i0 + r >= 0 && i0 + r < rows)
+                    col[r] = combine(tile[r][jl], alpha, beta, &old[q], BETA ? 2 : mode);
             }
         }
         __syncthreads();
@@ -334,8 +363,13 @@ template <int TR, int TC, bool SHIFT>
 void launch_transpose(int64_t rows, int64_t cols, double alpha, const double *src, int64_t lds, double beta,
                       double *dst, int64_t ldd, int mode, hipStream_t s) {
     const int64_t nx = (rows + (SHIFT ? LINE : 0) + TR - 1) / TR, tiles = nx * ((cols + TC - 1) / TC);
-    hipLaunchKernelGGL((transpose_kernel<TR, TC, SHIFT>), dim3((unsigned)std::min<int64_t>(tiles, 1 << 23)), dim3(NT),
-                       0, s, rows, cols, alpha, src, lds, beta, dst, ldd, mode, (uint32_t)nx, (uint32_t)tiles);
+    const dim3 grid((unsigned)std::min<int64_t>(tiles, 1 << 23));
+#define CA_TRANSPOSE(BETA)                                                                                          \
+    hipLaunchKernelGGL((transpose_kernel<TR, TC, SHIFT, BETA>), grid, dim3(NT), 0, s, rows, cols, alpha, src, lds, beta, \
+                       dst, ldd, mode, (uint32_t)nx, (uint32_t)tiles)
+    if (mode == 2) CA_TRANSPOSE(true);
+    else CA_TRANSPOSE(false);
+#undef CA_TRANSPOSE
 }
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
