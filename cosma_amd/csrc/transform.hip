@@ -15,8 +15,8 @@
 // copies and the large transposes give every column of dst its own row
 // window, which starts where a line does, and use 16-byte accesses at the
 // 8-byte alignment of a double (8191 x 12289, ld 12291 / 8193: 'T' 421 us
-// element by element, 358 us in 16-byte accesses, 298 us in shifted windows =
-// 5.4 TB/s; 'N' 351 -> 250 us = 6.4 TB/s).
+// element by element, 358 us in 16-byte accesses, 283 us in shifted windows =
+// 5.7 TB/s; 'N' 351 -> 250 us = 6.4 TB/s).
 //
 // op = 'N': a workgroup covers 512 rows of one or two columns, a thread two
 //           consecutive doubles of each.
@@ -325,34 +325,43 @@ __global__ __launch_bounds__(NT) void transpose_kernel(int64_t rows, int64_t col
             }
         } else {
             // Edge tile: by element, from addresses clamped into the matrix so
-            // that no load waits for another (one element at a time, two edge
-            // tiles in 24 made 2601 x 12501 take 308 us with beta = 1/2).
+            // that a batch of loads is in flight together (one element at a time, two edge
+            // tiles in 24 made 2601 x 12501 take 308 us with beta = 1/2, 177 us in
+            // batches of 8, 152 us in one; without beta, whose tiles need fewer
+            // registers, batches keep 8191 x 12289 at 283 us, one batch 322 us).
             constexpr int IN = LR * TC / NT, OUT = TR * TC / NT;
-            double v[IN], old[OUT];
+            constexpr int UI = BETA ? IN : 8, UO = BETA ? OUT : OUT % 7 == 0 ? 7 : 8;   // loads per batch
+            static_assert(IN % UI == 0 && OUT % UO == 0, "whole batches");
+#pragma unroll 1
+            for (int e0 = t; e0 < LR * TC; e0 += NT * UI) {
+                double v[UI];
 #pragma unroll
-            for (int q = 0; q < IN; ++q) {
-                const int e = t + NT * q;
-                const int64_t i = min(max(i0 + e / TC, (int64_t)0), rows - 1), j = min(j0 + e % TC, cols - 1);
-                v[q] = src[j + i * lds];
-            }
-            if (BETA) {
-#pragma unroll
-                for (int q = 0; q < OUT; ++q) {
-                    const int e = t + NT * q;
-                    double *col = dst + min(j0 + e / TR, cols - 1) * ldd;
-                    old[q] = col[min(max(i0 + e % TR + shift(col + i0), (int64_t)0), rows - 1)];
+                for (int q = 0; q < UI; ++q) {
+                    const int e = e0 + NT * q;
+                    const int64_t i = min(max(i0 + e / TC, (int64_t)0), rows - 1), j = min(j0 + e % TC, cols - 1);
+                    v[q] = src[j + i * lds];
                 }
+#pragma unroll
+                for (int q = 0; q < UI; ++q) tile[(e0 + NT * q) / TC][(e0 + NT * q) % TC] = v[q];
             }
-#pragma unroll
-            for (int q = 0; q < IN; ++q) tile[(t + NT * q) / TC][(t + NT * q) % TC] = v[q];
             __syncthreads();
+#pragma unroll 1
+            for (int e0 = t; e0 < TR * TC; e0 += NT * UO) {
+                double old[UO];
 #pragma unroll
-            for (int q = 0; q < OUT; ++q) {
-                const int e = t + NT * q, jl = e / TR;
-                double *col = dst + (j0 + jl) * ldd + i0;
-                const int r = e % TR + shift(col);
-                if (j0 + jl < cols && i0 + r >= 0 && i0 + r < rows)
-                    col[r] = combine(tile[r][jl], alpha, beta, &old[q], BETA ? 2 : mode);
+                for (int q = 0; q < UO; ++q) {
+                    const int e = e0 + NT * q;
+                    double *col = dst + min(j0 + e / TR, cols - 1) * ldd;
+                    old[q] = BETA ? col[min(max(i0 + e % TR + shift(col + i0), (int64_t)0), rows - 1)] : 0.0;
+                }
+#pragma unroll
+                for (int q = 0; q < UO; ++q) {
+                    const int e = e0 + NT * q, jl = e / TR;
+                    double *col = dst + (j0 + jl) * ldd + i0;
+                    const int r = e % TR + shift(col);
+                    if (j0 + jl < cols && i0 + r >= 0 && i0 + r < rows)
+                        col[r] = combine(tile[r][jl], alpha, beta, &old[q], BETA ? 2 : mode);
+                }
             }
         }
         __syncthreads();
@@ -387,9 +396,10 @@ int launch_block_transform(char op, int64_t rows, int64_t cols, double alpha,
     const bool in_phase = ldd % LINE == 0 && phase_of(dst) == 0;   // every column of dst starts at a line
     const bool src_in_phase = lds % LINE == 0 && phase_of(src) == 0;
     // src and dst together exceed the 256 MB last-level cache, which hides
-    // shared lines (8191 x 12289 'T': 421 us, in shifted windows 298 us, 5000 x
-    // 5001: 111 and 79 us, but 3000 x 5000: 46 and 53 us)
+    // shared lines (8191 x 12289 'T': 421 us, in shifted windows 283 us, 5000 x
+    // 5001: 111 and 79 us, with beta = 1/2 157 and 116 us, but 3000 x 5000: 46 and 53 us)
     const bool large = rows * cols >= 20000000;
+    const bool vec = aligned16(src) && aligned16(dst) && (lds % 2 == 0) && (ldd % 2 == 0);
     if (op == 'N') {
         // a 512-row window would leave most threads idle (40 x 100000: 25 -> 15 us;
         // 1 x 10^8: 9.2 -> 2.4 ms, 240 x 2000000: 1.91 -> 1.53 ms)
@@ -417,7 +427,11 @@ int launch_block_transform(char op, int64_t rows, int64_t cols, double alpha,
         // both sides in whole lines (16384^2: 769 us in 64 x 64 tiles, 700 us;
         // slower below 4096 rows, 2000 x 16000: 90 and 112 us)
         launch_transpose<128, 64, false>(rows, cols, alpha, src, lds, beta, dst, ldd, mode, s);
-    } else if (!(in_phase && src_in_phase) && large && rows >= 1024 && cols >= 1024) {
+    } else if (!(in_phase && (src_in_phase || (vec && (mode != 2 || rows * cols < 32000000)))) && large && rows >= 1024 &&
+               cols >= 1024) {
+        // with dst in whole lines the windows' extra columns buy nothing until
+        // dst is also read from beyond the cache (2000 x 30002: 177 us in 64 x
+        // 64 tiles, 195 us; with beta = 1/2 410 and 272 us, 4096 x 6002: 103 and 110 us)
         launch_transpose<112, 64, true>(rows, cols, alpha, src, lds, beta, dst, ldd, mode, s);
     } else {
         const int64_t bx = (rows + TT - 1) / TT;
@@ -427,7 +441,6 @@ int launch_block_transform(char op, int64_t rows, int64_t cols, double alpha,
             set_error("block_transform: %lld rows exceed the grid limit", (long long)rows);
             return COSMA_AMD_ERR_UNSUPPORTED;
         }
-        const bool vec = aligned16(src) && aligned16(dst) && (lds % 2 == 0) && (ldd % 2 == 0);
         // with plenty of workgroups, four tiles each (the vectorised kernel
         // prefetches the next tile of a workgroup during the current one)
         if (vec && bx * by > 4096) by = (by + 3) / 4;

@@ -27,6 +27,7 @@ def matrix(rows, cols, pad, offset, seed):
     ("N", 1, (1 << 23) + 1, 0, 1, 0, 0), ("N", 3, (1 << 24) - 1, 1, 0, 1, 1),             # narrow, cut in pieces
     ("T", 1024, 19532, 1, 0, 0, 1), ("T", 5001, 4003, 0, 1, 1, 0), ("T", 19532, 1024, 0, 0, 0, 0),   # shifted
     ("T", 4096, 16384, 0, 0, 0, 0), ("T", 4111, 16401, 15, 1, 0, 0),                    # whole lines
+    ("T", 2601, 8501, 1, 0, 1, 0), ("T", 1040, 30802, 0, 0, 0, 0), ("T", 1040, 30702, 0, 0, 0, 0),   # part tiles; dst in whole lines
 ])
 def test_transform_forms(handle, op, rows, cols, pad_src, pad_dst, off_src, off_dst, alpha, beta):
     import torch
