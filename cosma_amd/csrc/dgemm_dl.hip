@@ -40,12 +40,12 @@
 
 #include "common.hpp"
 #include "dgemm_dl.hpp"
+#include "dl_index.hpp"
 
 namespace cosma_amd {
 namespace {
 
 constexpr int BK = 16;       // k-step
-constexpr int NXCD = 8;
 
 typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));   // 16-byte access at 8-byte alignment
 
@@ -312,14 +312,9 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WP
     const double *__restrict__ B, int64_t ldb,
     double beta, double *__restrict__ C, int64_t ldc, int group_m) {
     __shared__ __attribute__((aligned(16))) double sm[NS * (BM + BN) * BK];
-    // ---- tile rasterisation (XCD-aware, grouped along m)
-    const uint32_t tiles_m = (uint32_t)((M + BM - 1) / BM), tiles_n = (uint32_t)((N + BN - 1) / BN);
-    const uint32_t T = gridDim.x, q8 = T / NXCD, r8 = T % NXCD, xcd = blockIdx.x % NXCD, loc = blockIdx.x / NXCD;
-    const uint32_t bid = xcd * q8 + min(xcd, r8) + loc;
-    const uint32_t per_group = group_m * tiles_n, grp = bid / per_group, in_group = bid - grp * per_group;
-    const uint32_t gsize = min((uint32_t)group_m, tiles_m - grp * group_m);
-    const int64_t m0 = (int64_t)(grp * group_m + in_group % gsize) * BM;
-    const int64_t n0 = (int64_t)(in_group / gsize) * BN;
+    const dl::TileAt t = dl::raster(blockIdx.x, gridDim.x, (uint32_t)((M + BM - 1) / BM),
+                                    (uint32_t)((N + BN - 1) / BN), (uint32_t)group_m);
+    const int64_t m0 = (int64_t)t.m * BM, n0 = (int64_t)t.n * BN;
     dl_tile<BM, BN, NS, WM, WN, AK, BKC, false>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, m0, n0, sm);
 }
 
@@ -364,10 +359,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 template <int BM, int BN, int NS, int WPE, int WM, int WN>
 void launch(char ta, char tb, int64_t m, int64_t n, int64_t k, double alpha, const double *a, int64_t lda,
             const double *b, int64_t ldb, double beta, double *c, int64_t ldc, int group_m, hipStream_t s) {
-    const dim3 grid((unsigned)(((m + BM - 1) / BM) * ((n + BN - 1) / BN))), block(64 * WM * WN);
+    const int64_t tiles_m = (m + BM - 1) / BM;
+    const dim3 grid((unsigned)(tiles_m * ((n + BN - 1) / BN))), block(64 * WM * WN);
+    const int rows = dl::clamp_group(group_m, tiles_m);
 #define CA_LAUNCH_DL(X, Y)                                                                                        \
     hipLaunchKernelGGL((dgemm_dl_kernel<BM, BN, NS, WPE, WM, WN, X, Y>), grid, block, 0, s, m, n, k, alpha, a, lda, b,   \
-                       ldb, beta, c, ldc, group_m)
+                       ldb, beta, c, ldc, rows)
     // template flags: operand k-contiguous (A 'T', B 'N')
     if (ta == 'T' && tb == 'N') CA_LAUNCH_DL(true, true);
     else if (ta == 'N' && tb == 'N') CA_LAUNCH_DL(false, true);
