@@ -19,8 +19,8 @@
 //     32768 TN, one 64 x 64 tile per CU: 1332 us with two stages, 1000 us with
 //     three).
 //   * Fragment registers are double-buffered by half-step, and each batch of
-//     reads is waited for before the next one is issued (by then 8 to 32
-//     MFMAs old).  Left to the compiler, the wait stood behind the next batch
+//     reads is waited for before the next one is issued (by then as many MFMAs
+//     old as a half-step holds: 16 per wave at 128 x 128, 2 at 32 x 32).  Left to the compiler, the wait stood behind the next batch
 //     and covered it too, idling the wave for an LDS round trip per half-step
 //     (8192^3 TN 70.6 -> 73.0 TF, NN 70.7 -> 72.1 with the scalar addresses).
 //   * LDS layout per operand and stage, every eight lanes of a fragment read on
@@ -45,7 +45,8 @@
 namespace cosma_amd {
 namespace {
 
-constexpr int BK = 16;       // k-step
+using dl::BK;
+using dl::row_swz;
 
 typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));   // 16-byte access at 8-byte alignment
 
@@ -53,9 +54,6 @@ typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));   // 16-b
 constexpr int wait_vm(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0F70; }
 constexpr int WAIT_LGKM0 = 0xC07F;
 constexpr int WAIT_VM0_LGKM0 = 0x0070;
-
-// Slot (of eight) of k-pair kp in row r of a k-contiguous tile is kp ^ row_swz(r).
-__device__ __forceinline__ int row_swz(int r) { return ((r >> 2) & 3) | ((r & 2) << 1); }
 
 template <int R, bool KCONTIG, int NW>
 struct Operand {
@@ -71,21 +69,14 @@ struct Operand {
 
     __device__ __forceinline__ Operand(const double *x, int64_t ld, int64_t r0, int64_t ext, int wave, int lane) {
         ldb = ld * 8;
-        const int last = (int)min((int64_t)(R - 1), ext - 1 - r0);   // last row of the tile inside the matrix
-        if (KCONTIG) {
-            base = reinterpret_cast<const char *>(x + r0 * ld);
+        const int last = dl::last_row<R>(ext, r0);
+        base = KCONTIG ? reinterpret_cast<const char *>(x + r0 * ld)
+                       : reinterpret_cast<const char *>(x + r0) + (int64_t)(wave * dl::K_PER_WAVE<R>) * ldb;
 #pragma unroll
-            for (int q = 0; q < LOADS; ++q) {
-                const int row = 8 * (wave + NW * q) + (lane >> 3);
-                off[q] = (uint32_t)min(row, last) * (uint32_t)ldb + (uint32_t)(((lane & 7) ^ row_swz(row)) * 16);
-            }
-        } else {
-            const int e = 2 * lane;                                  // position in the 128 doubles of an instruction
-            const int kl = e / R, pos = e % R;
-            const int odd_kp = R == 128 ? (wave >> 1) & 1 : R == 64 ? wave & 1 : lane >> 5;
-            const int row = min(pos ^ (16 * odd_kp), last & ~1);
-            base = reinterpret_cast<const char *>(x + r0) + (int64_t)(wave * (128 / R)) * ldb;
-            off[0] = (uint32_t)kl * (uint32_t)ldb + (uint32_t)row * 8;
+        for (int q = 0; q < NOFF; ++q) {
+            const dl::Element e = dl::lane_load<R, KCONTIG, NW>(q, wave, lane, last);
+            off[q] = KCONTIG ? (uint32_t)e.row * (uint32_t)ldb + (uint32_t)e.k * 8
+                             : (uint32_t)e.k * (uint32_t)ldb + (uint32_t)e.row * 8;
         }
     }
     __device__ __forceinline__ void issue(int k0, double *tile, int wave) const {
@@ -93,7 +84,7 @@ struct Operand {
         for (int q = 0; q < LOADS; ++q) {
             // scalar base + 32-bit lane offset (the asm keeps the compiler from
             // folding the lane offset into 64-bit vector adds per load)
-            const char *u = KCONTIG ? base + (int64_t)k0 * 8 : base + (int64_t)(k0 + q * (128 * NW / R)) * ldb;
+            const char *u = KCONTIG ? base + (int64_t)k0 * 8 : base + (int64_t)(k0 + q * dl::K_PER_ROUND<R, NW>) * ldb;
             asm("" : "+s"(u));
             __builtin_amdgcn_global_load_lds(static_cast<const void *>(u + off[KCONTIG ? q : 0]),
                                              (__attribute__((address_space(3))) void *)(tile + 128 * (wave + NW * q)),
@@ -108,7 +99,7 @@ struct Operand {
     }
     __device__ __forceinline__ static void tail_load(const double *x, int64_t ld, int64_t r0, int64_t ext, int64_t k0,
                                                      int kt, double (&v)[TAIL]) {
-        const int last = (int)min((int64_t)(R - 1), ext - 1 - r0);
+        const int last = dl::last_row<R>(ext, r0);
 #pragma unroll
         for (int e = 0; e < TAIL; ++e) {
             int row, k;
@@ -172,11 +163,7 @@ __device__ __forceinline__ void dl_tile(int64_t M, int64_t N, int64_t K, double 
     const Frag<BM, AK, FM> fra(wm * (BM / WM) + 4 * (li & 3) + (li >> 2), g);
     const Frag<BN, BKC, FN> frb(wn * (BN / WN) + li, g);
 
-    // Full steps; a row-contiguous operand with an odd extent keeps the last
-    // k out of them (the 16-byte load of its last row reads one element
-    // beyond the row, which only inside the matrix is the next column's).
-    const bool hold_last = (!AK && (M & 1)) || (!BKC && (N & 1));
-    const int nk = (int)((hold_last ? K - 1 : K) / BK);
+    const int nk = dl::full_steps(M, N, K, AK, BKC);
     const int kt = (int)(K - (int64_t)nk * BK);   // 0..16
     double ta[OA::TAIL], tb[OB::TAIL];
     auto tail_load = [&]() {

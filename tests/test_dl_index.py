@@ -26,3 +26,10 @@ def run(exe, what):
 def test_every_group_m_walks_every_tile_once(exe):
     """cosma_amd_dgemm_set_tuning takes any group_m >= 0; the kernel's 32-bit walk is right for all of them."""
     assert run(exe, "raster").count("ok raster") == 8 * 14
+
+
+def test_loads_end_inside_the_operand(exe):
+    """For odd and even extents, every k up to three steps and the tightest leading dimension, as A and as B; the
+    over-read that the steps would make of an odd row-contiguous operand without holding back its last k is seen."""
+    out = run(exe, "loads")
+    assert [out.count(s) for s in ("ok loads inside", "ok loads complete", "ok over-read seen")] == [10, 10, 10]
