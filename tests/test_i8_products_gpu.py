@@ -25,3 +25,23 @@ def test_int8_products_equal_bf16_products(handle, m, n, k, ta, tb):
         assert info["method"] == method
         out.append(C)
     assert torch.isfinite(out[0]).all() and torch.equal(out[0], out[1])
+
+
+def test_int8_products_of_planes_beyond_the_last_level_cache(handle):
+    """Planes of more than 384 Mi elements take another INT8 kernel: just past that line, with ragged tiles."""
+    import torch
+    import cosma_amd as ca
+    m, n, k = 257, 12300, 32768
+    assert (m + n) * k > 384 << 20
+    g = torch.Generator(device="cuda").manual_seed(11)
+    A = torch.randn(m, k, dtype=torch.float64, device="cuda", generator=g)   # op(A) = A^T: rows contiguous in k
+    B = torch.randn(n, k, dtype=torch.float64, device="cuda", generator=g)
+    out = []
+    for method in (ca.OZAKI_MODULI, ca.OZAKI_MODULI_BF16):
+        C = torch.full((n, m), float("nan"), dtype=torch.float64, device="cuda")
+        info = handle.dgemm_ozaki("T", "N", m, n, k, 1.0, A.data_ptr(), k, B.data_ptr(), k, 0.0, C.data_ptr(), m,
+                                  method=method, count=16)
+        torch.cuda.synchronize()
+        assert info["method"] == method
+        out.append(C)
+    assert torch.isfinite(out[0]).all() and torch.equal(out[0], out[1])
