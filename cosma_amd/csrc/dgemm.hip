@@ -743,7 +743,7 @@ int grouped_tile_shape(int cfg, int *bm, int *bn) {
     case 2: *bm = 128; *bn = 64; return COSMA_AMD_OK;
     case 3: *bm = 128; *bn = 128; return COSMA_AMD_OK;
     case 4: *bm = 64; *bn = 64; return COSMA_AMD_OK;   // direct: one wave per tile, no LDS
-    case 5: *bm = 32; *bn = 32; return COSMA_AMD_OK;   // direct, 32 x 32
+    case 5: *bm = 32; *bn = 32; return COSMA_AMD_OK;   // LDS-staged; direct in plans beyond the direct-LDS kernels
     default:
         set_error("grouped dgemm: unknown tile configuration %d", cfg);
         return COSMA_AMD_ERR_INVALID_ARG;

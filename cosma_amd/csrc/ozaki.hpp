@@ -25,9 +25,10 @@ constexpr double kGroupInverse[4] = {1.0 / kGroupProduct[0], 1.0 / kGroupProduct
 // limb sum of 20 terms |c_l| * w < 20 * 2^7 * 2^41 < 2^53 stays exact in FP64.
 constexpr int LIMB = 41;
 constexpr int NLIMB = 4;
-// Largest P (bits of the integer inputs) for which the residues stay exact:
-// a' / m_l < 2^51 for every modulus (>= 173) keeps the split's FP64 quotient
-// within one of the true one, so a single correction step is exact.
+// Largest P (bits of the integer inputs) for which the residues are taken: the
+// quotients by the group products stay below 2^44 (the last group, 179 * 173 =
+// 2^14.9, has 2^43.1), where FP64 quotients are within 2^-8 of the true ones, so
+// that one reduction leaves a rest below 2^48 (moduli_residues16).
 constexpr int MAX_P = 58;
 // Exponent given to an all-zero row or column: its entries and products are
 // zero whatever the scaling, and it drops out of the error estimate.

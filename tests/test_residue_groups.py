@@ -36,3 +36,14 @@ def test_group_reduction_gives_symmetric_residues():
                     want = x % m
                     want = want - m if want > (m - 1) // 2 else want
                     assert residue(y, m) == want, (P, x, m)
+
+
+def test_the_header_holds_the_constants_checked_here():
+    import os
+    import re
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    text = open(os.path.join(root, "cosma_amd", "csrc", "ozaki.hpp")).read()
+    moduli = re.search(r"kModuli\[20\] = \{([^}]*)\}", text).group(1)
+    assert [int(x) for x in moduli.split(",")] == MODULI
+    assert int(re.search(r"constexpr int MOD_GROUP = (\d+);", text).group(1)) == GROUP
+    assert int(re.search(r"constexpr int MAX_P = (\d+);", text).group(1)) == 58   # the largest P above
