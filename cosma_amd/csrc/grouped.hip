@@ -140,7 +140,8 @@ int grouped_create(cosma_amd_handle_t h, const cosma_amd_gemm_desc *d, int64_t c
     }
     p->h = h;
     p->nprob = (int)probs.size();
-    p->signature = fnv(sig, (uint64_t)probs.size());
+    // which kernels a configuration names depends on dl as well
+    p->signature = fnv(fnv(sig, (uint64_t)probs.size()), p->dl >= 0);
     int rc = COSMA_AMD_OK;
     for (int cfg : {1, 2, 3, 5}) {
         if (rc != COSMA_AMD_OK) break;

@@ -71,3 +71,23 @@ def test_leading_dimension_beyond_the_lane_offsets(handle):
     B[:, :k] = torch.rand((n, k), dtype=torch.float64, device="cuda", generator=g)
     probs.append(("N", "N", m, n, k, 1.0, tensor(m, k, 0, g), B, 0.0, tensor(m, n, 0, g)))
     check(handle, probs, (1, 2, 3, 4, 5))
+
+
+def test_tuned_choice_is_not_taken_over_by_other_kernels(handle):
+    """A plan beyond the direct-LDS kernels runs others under the same configuration numbers: what tuning found for
+    the same shapes within their limits is not its choice."""
+    import torch
+    import cosma_amd as ca
+    m, count, ld = 16, 20000, (1 << 22) + 2
+    A = torch.rand((m, m), dtype=torch.float64, device="cuda")
+    B = torch.zeros((m, ld), dtype=torch.float64, device="cuda")
+    C = torch.zeros(count * m * m, dtype=torch.float64, device="cuda")
+
+    def plan(ldb, cfg=0):
+        return ca.Grouped(handle, [("N", "N", m, m, m, 1.0, A.data_ptr(), m, B.data_ptr(), ldb if i == 0 else m, 0.0,
+                                    C.data_ptr() + 8 * i * m * m, m) for i in range(count)], tile_config=cfg)
+
+    first = plan(m)
+    first.tune()
+    assert plan(m).info() == first.info()
+    assert plan(ld).info() == plan(ld, 1).info()   # the default: 64 x 64 with its default grid
