@@ -83,6 +83,7 @@ Kind classify(const void *p) {
 constexpr size_t SLOT_BYTES = 64ull << 20;   // pinned staging slot
 constexpr int N_SLOTS = 4;                   // per direction
 constexpr int64_t C_SLOTS = 4;               // device slots of incoming C tiles
+constexpr int64_t PACK_ELEMENTS = (int64_t)1 << 21;   // smallest block that a pageable operand is cut into (16 MB)
 
 int grow(DevBuf &b, size_t bytes) {
     if (b.bytes >= bytes) return COSMA_AMD_OK;
@@ -631,11 +632,22 @@ static int stream_dgemm_body(cosma_amd_handle_t h, char ta, char tb, int64_t m, 
         // Four slots of tiles rounded up to 128 can hold more than one coarse
         // tile's slot (1793 x 1793: 34 MB and 26 MB): only within the budget.
         const int64_t rm = resident_tile(tm, m), rn = resident_tile(tn, n);
+        const int64_t rk = resident_tile(tk, k);
         const int64_t slots = std::min<int64_t>(C_SLOTS, ((m + rm - 1) / rm) * ((n + rn - 1) / rn));
-        if (!defer_c || needA + needB + needC + (size_t)slots * rm * rn * 8 <= limit) {
+        const bool fits = !defer_c || needA + needB + needC + (size_t)slots * rm * rn * 8 <= limit;
+        // Pageable blocks are packed on the host, with a thread per 4 MB: they are
+        // cut only where at least four threads remain, and not with a C that is
+        // packed on its way up as well (all operands pageable, 3000^3: 6.5 ms in
+        // 5000^3 tiles, 11.7 ms in 1024^3 with two threads a block; 8192^3, 2048^3
+        // tiles: 37.6 and 34.4 ms, with beta = 1/2 42.3 and 47.1 ms).
+        auto packs = [](Kind kind, int64_t coarse, int64_t finer) {
+            return kind != PAGEABLE || finer >= PACK_ELEMENTS || finer == coarse;
+        };
+        if (fits && packs(A.kind, tm * tk, rm * rk) && packs(B.kind, tk * tn, rk * rn) && packs(kc, tm * tn, rm * rn) &&
+            !(defer_c && kc == PAGEABLE)) {
             fm = rm;
             fn = rn;
-            fk = resident_tile(tk, k);
+            fk = rk;
         }
     }
     int rc = resident ? stream_resident(h, A, B, kc, m, n, k, alpha, beta, c, ldc, copy_c_back,

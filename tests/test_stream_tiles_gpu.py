@@ -65,3 +65,49 @@ def test_finer_tiles_keep_to_the_memory_limit():
         assert e.value.status == 3
     finally:
         ca.fail_allocations(0, 0)
+
+
+TILES_OF = """
+import torch, sys
+import cosma_amd as ca
+h = ca.Handle(0)
+def call(kinds, m, n, k, beta):
+    put = {"d": lambda t: t.cuda(), "p": lambda t: t.pin_memory(), "g": lambda t: t}
+    A, B, C = (put[x](torch.zeros(s, dtype=torch.float64)) for x, s in zip(kinds, ((k, m), (n, k), (n, m))))
+    print("call", kinds, m, n, k, beta, file=sys.stderr, flush=True)
+    h.dgemm_host("N", "N", m, n, k, 1.0, A.data_ptr(), m, B.data_ptr(), k, beta, C.data_ptr(), m)
+for beta in (0.0, 0.5):
+    for kinds in ("ppp", "gpp", "pgp", "ppg", "ddg", "ddp"):
+        call(kinds, 1800, 1800, 1800, beta)
+    call("ddg", 8192, 8192, 64, beta)
+    call("dgp", 1500, 7000, 1200, beta)
+    call("gdp", 1500, 7000, 1200, beta)
+"""
+
+
+def test_pageable_blocks_stay_large_enough_for_the_packing_threads():
+    """The traced tiles of host products: 1800^3 is cut in 2 x 2 tiles of C unless an operand is pageable (its blocks
+    of 1024^2 would be packed by two threads).  Pageable operands whose blocks keep 16 MB or their size are cut,
+    unless beta != 0 has a pageable C packed on its way up too."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", TILES_OF], cwd=root, capture_output=True, text=True, timeout=100,
+                       env={**os.environ, "COSMA_AMD_TRACE": "1"})
+    assert r.returncode == 0, r.stderr[-2000:]
+    tiles, got = {}, None
+    for line in r.stderr.splitlines():
+        if line.startswith("call "):
+            got = tuple(line.split()[1:])
+            tiles[got] = 0
+        elif line.startswith("[cosma_amd] tile ("):
+            tiles[got] += 1
+    want = {}
+    for beta in ("0.0", "0.5"):
+        for kinds in ("ppp", "gpp", "pgp", "ppg", "ddg", "ddp"):
+            want[kinds, "1800", "1800", "1800", beta] = 1 if "g" in kinds else 4
+        want["ddg", "8192", "8192", "64", beta] = 16 if beta == "0.0" else 4
+        for kinds in ("dgp", "gdp"):   # B in blocks of 1200 x 1792, A in one
+            want[kinds, "1500", "7000", "1200", beta] = 4
+    assert tiles == want
