@@ -72,6 +72,7 @@ __global__ __launch_bounds__(NT) void copy_kernel(int64_t rows, int64_t cols, do
         return STREAM ? __builtin_nontemporal_load(q) : *q;
     };
     const int64_t r0 = 2 * ((int64_t)blockIdx.x * NT + threadIdx.x);
+    if (r0 - (SHIFT ? LINE - 1 : 0) >= rows) return;   // no row of any column (3 x 300000: 84 us with these waves in the loop, 59 us)
     for (int64_t c0 = U * (int64_t)blockIdx.y; c0 < cols; c0 += U * (int64_t)gridDim.y) {
         f64x2u v[U], old[U];
         int64_t r[U];
@@ -401,9 +402,12 @@ int launch_block_transform(char op, int64_t rows, int64_t cols, double alpha,
     const bool large = rows * cols >= 20000000;
     const bool vec = aligned16(src) && aligned16(dst) && (lds % 2 == 0) && (ldd % 2 == 0);
     if (op == 'N') {
-        // a 512-row window would leave most threads idle (40 x 100000: 25 -> 15 us;
-        // 1 x 10^8: 9.2 -> 2.4 ms, 240 x 2000000: 1.91 -> 1.53 ms)
-        if (rows <= NT && rows * cols >= (1 << 20)) {
+        // Many columns of few rows: a workgroup per two columns leaves most of
+        // its threads idle, but what counts up to some 2^14 columns is that
+        // there are many (33 x 7943: 4.2 us, 6.9 us as a list, x 31775: 9.6 and
+        // 8.2 us; 1 x 10^8: 9.2 and 2.4 ms).  Fuller windows are as fast (128 x
+        // 65536: 22.1 and 21.4 us, with beta = 1/2 33.3 and 37.1 us).
+        if (rows <= (mode == 2 ? 48 : 64) && cols >= (1 << 14) + rows * (1 << 7)) {
             const CopyBlock one{src, dst, lds, ldd, rows, cols};
             return launch_block_copies(&one, 1, alpha, beta, s);
         }
