@@ -56,21 +56,23 @@ __device__ __forceinline__ f64x2u combine2(f64x2u x, double alpha, double beta, 
 // Position of an element in its 128-byte line.
 __device__ __forceinline__ int phase(const double *p) { return (int)(reinterpret_cast<uintptr_t>(p) >> 3) & (LINE - 1); }
 
+// 16-byte load, streaming past the caches or not.
+template <bool NONTEMPORAL>
+__device__ __forceinline__ f64x2u load2(const double *p) {
+    const f64x2u *q = reinterpret_cast<const f64x2u *>(p);
+    return NONTEMPORAL ? __builtin_nontemporal_load(q) : *q;
+}
+
 // dst(rows x cols) <- f(src(rows x cols)).  Grid: x over 512-row windows, y
-// over columns or pairs of columns.  SHIFT: row windows by dst's lines.
-// STREAM, for operands beyond the last-level cache: one 16-byte piece per
-// thread, all accesses non-temporal (16384^2, beta = 1/2: 1052 -> 992 us;
-// with two pieces 1002 us).  Otherwise two pieces, loaded before either is
-// stored, and cached loads (3000 x 5000: 41 -> 36 us).
-template <bool SHIFT, bool STREAM>
+// over groups of U columns.  SHIFT: row windows by dst's lines.  SRC_NT,
+// DST_NT: loads that stream past the caches (streamed()); the stores always do.
+// U pieces per thread are loaded before one is stored: two, but one where all
+// streams, except from short columns and from so many that a workgroup walks
+// several (10000 x 13400, beta = 1/2: 539 and 518 us; 300 x 446666: 564 and 620 us).
+template <bool SHIFT, bool SRC_NT, bool DST_NT, int U>
 __global__ __launch_bounds__(NT) void copy_kernel(int64_t rows, int64_t cols, double alpha,
                                                   const double *__restrict__ src, int64_t lds, double beta,
                                                   double *__restrict__ dst, int64_t ldd, int mode) {
-    constexpr int U = STREAM ? 1 : 2;
-    auto load2 = [](const double *p) {
-        const f64x2u *q = reinterpret_cast<const f64x2u *>(p);
-        return STREAM ? __builtin_nontemporal_load(q) : *q;
-    };
     const int64_t r0 = 2 * ((int64_t)blockIdx.x * NT + threadIdx.x);
     if (r0 - (SHIFT ? LINE - 1 : 0) >= rows) return;   // no row of any column (3 x 300000: 84 us with these waves in the loop, 59 us)
     for (int64_t c0 = U * (int64_t)blockIdx.y; c0 < cols; c0 += U * (int64_t)gridDim.y) {
@@ -83,8 +85,8 @@ __global__ __launch_bounds__(NT) void copy_kernel(int64_t rows, int64_t cols, do
             r[u] = r0 - (SHIFT ? phase(dst + c * ldd) : 0);
             in[u] = c < cols && r[u] >= 0 && r[u] + 1 < rows;
             if (!in[u]) continue;
-            v[u] = load2(src + r[u] + c * lds);
-            if (mode == 2) old[u] = load2(dst + r[u] + c * ldd);
+            v[u] = load2<SRC_NT>(src + r[u] + c * lds);
+            if (mode == 2) old[u] = load2<DST_NT>(dst + r[u] + c * ldd);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -119,6 +121,7 @@ struct BlockList {
     } b[LIST];
     int n;
 };
+template <bool SRC_NT, bool DST_NT>
 __global__ __launch_bounds__(NT) void copy_list_kernel(BlockList list, double alpha, double beta, int mode) {
     int lo = 0, hi = list.n - 1;   // last block with first <= this workgroup
     while (lo < hi) {
@@ -141,8 +144,8 @@ __global__ __launch_bounds__(NT) void copy_list_kernel(BlockList list, double al
         r[q] = (int)(2 * (idx - (uint32_t)c[q] * pairs)) - phase(dst + c[q] * ldd);
         in[q] = c[q] < cols && r[q] >= 0 && r[q] + 1 < rows;
         if (!in[q]) continue;
-        v[q] = *reinterpret_cast<const f64x2u *>(src + r[q] + c[q] * lds);
-        if (mode == 2) old[q] = *reinterpret_cast<const f64x2u *>(dst + r[q] + c[q] * ldd);
+        v[q] = load2<SRC_NT>(src + r[q] + c[q] * lds);
+        if (mode == 2) old[q] = load2<DST_NT>(dst + r[q] + c[q] * ldd);
     }
 #pragma unroll
     for (int q = 0; q < ITEMS; ++q) {
@@ -385,6 +388,20 @@ void launch_transpose(int64_t rows, int64_t cols, double alpha, const double *sr
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 inline int phase_of(const void *p) { return (int)(reinterpret_cast<uintptr_t>(p) & (8 * LINE - 1)); }   // bytes into its line
 
+// Which loads of a copy of so many elements stream past the 256 MB last-level
+// cache: none while it holds what is read, src's while it still holds dst, else
+// both (1000 x 20000: 51.6 us streamed, 46.4 us cached, 1000 x 50000: 127 and
+// 135 us; with beta = 1/2, 4096 x 4882: 73 us streamed, 67.5 us cached, 1000 x
+// 30000: 116 and 128 us, 104 us with src streamed, 3000 x 15000: 186 us so, 163
+// us all streamed).
+struct Streamed {
+    bool src, dst;
+};
+Streamed streamed(int64_t elements, int mode) {
+    if (mode != 2) return {elements >= 38000000, elements >= 38000000};
+    return {elements >= 21000000, elements >= 34000000};
+}
+
 int mode_of(double alpha, double beta) { return (alpha == 1.0 && beta == 0.0) ? 0 : (beta == 0.0 ? 1 : 2); }
 
 }  // namespace
@@ -411,21 +428,27 @@ int launch_block_transform(char op, int64_t rows, int64_t cols, double alpha,
             const CopyBlock one{src, dst, lds, ldd, rows, cols};
             return launch_block_copies(&one, 1, alpha, beta, s);
         }
-        const bool shift = !in_phase && rows >= 1024, stream = rows * cols >= (1 << 24);
+        const bool shift = !in_phase && rows >= 1024;
+        const Streamed st = streamed(rows * cols, mode);
         const int64_t bx = (rows + (shift ? LINE - 1 : 0) + 2 * NT - 1) / (2 * NT);
-        const int64_t by = std::min<int64_t>(stream ? cols : (cols + 1) / 2, 65535);
+        const int u = st.dst && rows >= 3 * NT / 2 && cols <= 100000 ? 1 : 2;
+        const int64_t by = std::min<int64_t>((cols + u - 1) / u, 65535);
         if (bx > 0x7fffffffLL) {
             set_error("block_transform: %lld rows exceed the grid limit", (long long)rows);
             return COSMA_AMD_ERR_UNSUPPORTED;
         }
         const dim3 grid((unsigned)bx, (unsigned)by);
-#define CA_COPY(SHIFT, STREAM)                                                                                       \
-    hipLaunchKernelGGL((copy_kernel<SHIFT, STREAM>), grid, dim3(NT), 0, s, rows, cols, alpha, src, lds, beta, dst, \
-                       ldd, mode)
-        if (shift && stream) CA_COPY(true, true);
-        else if (shift) CA_COPY(true, false);
-        else if (stream) CA_COPY(false, true);
-        else CA_COPY(false, false);
+#define CA_COPY(SHIFT, SRC_NT, DST_NT, U)                                                                            \
+    hipLaunchKernelGGL((copy_kernel<SHIFT, SRC_NT, DST_NT, U>), grid, dim3(NT), 0, s, rows, cols, alpha, src, lds,  \
+                       beta, dst, ldd, mode)
+        if (u == 1 && shift) CA_COPY(true, true, true, 1);
+        else if (u == 1) CA_COPY(false, true, true, 1);
+        else if (st.dst && shift) CA_COPY(true, true, true, 2);
+        else if (st.dst) CA_COPY(false, true, true, 2);
+        else if (st.src && shift) CA_COPY(true, true, false, 2);
+        else if (st.src) CA_COPY(false, true, false, 2);
+        else if (shift) CA_COPY(true, false, false, 2);
+        else CA_COPY(false, false, false, 2);
 #undef CA_COPY
     } else if (in_phase && src_in_phase && rows >= 4096 && rows * cols >= ((int64_t)1 << 26)) {
         // both sides in whole lines (16384^2: 769 us in 64 x 64 tiles, 700 us;
@@ -464,9 +487,18 @@ int launch_block_copies(const CopyBlock *blocks, int64_t n, double alpha, double
     BlockList list;
     list.n = 0;
     uint32_t groups = 0;
+    int64_t elements = 0;   // of the blocks that read whole lines; others share them (33 x 2033601: 228 us cached, 364 us)
+    for (int64_t i = 0; i < n; ++i)
+        if (blocks[i].rows >= NT / 2) elements += blocks[i].rows * blocks[i].cols;
+    const Streamed st = streamed(elements, mode);
     auto flush = [&]() -> int {
         if (list.n == 0) return COSMA_AMD_OK;
-        hipLaunchKernelGGL(copy_list_kernel, dim3(groups), dim3(NT), 0, s, list, alpha, beta, mode);
+#define CA_LIST(SRC_NT, DST_NT) \
+    hipLaunchKernelGGL((copy_list_kernel<SRC_NT, DST_NT>), dim3(groups), dim3(NT), 0, s, list, alpha, beta, mode)
+        if (st.dst) CA_LIST(true, true);
+        else if (st.src) CA_LIST(true, false);
+        else CA_LIST(false, false);
+#undef CA_LIST
         CA_HIP(hipGetLastError());
         list.n = 0;
         groups = 0;
