@@ -355,7 +355,10 @@ __global__ __launch_bounds__(256) void gz_gamma(const OzProblem *probs, const in
 // along the vector, so the residue stores are contiguous runs.  Strided
 // operand: 64 x 64 (vector x k) tiles are read along the vectors into LDS and
 // transposed, four threads per vector writing 64 contiguous bytes per plane.
-__global__ __launch_bounds__(256) void gz_split(const OzProblem *probs, const int *pbits, GzModuli md) {
+// Held to 128 registers, four waves per SIMD, by which it is bound: the residues
+// of wide integers alone would take 150 (64 problems of 200 to 600, 10 moduli:
+// 257 us, 230 us with four waves).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void gz_split(const OzProblem *probs, const int *pbits, GzModuli md) {
     const OzProblem &q = probs[blockIdx.x];
     if (q.scale_only) return;
     const int P = pbits[blockIdx.x];
