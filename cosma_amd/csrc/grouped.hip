@@ -143,43 +143,39 @@ int grouped_create(cosma_amd_handle_t h, const cosma_amd_gemm_desc *d, int64_t c
     // which kernels a configuration names depends on dl as well
     p->signature = fnv(fnv(sig, (uint64_t)probs.size()), p->dl >= 0);
     int rc = COSMA_AMD_OK;
+    // A configuration's descriptors, then their first tile indices (the kernels'
+    // search array), then the owner of every tile (direct-LDS kernels), in one
+    // upload: a copy each cost a plan of 64 problems 110 us of 226.
+    const size_t n = probs.size(), dbytes = n * sizeof(GroupedProblem), sbytes = n * sizeof(int64_t);
+    std::vector<char> image;
     for (int cfg : {1, 2, 3, 5}) {
         if (rc != COSMA_AMD_OK) break;
         int bm, bn;
         grouped_tile_shape(cfg, &bm, &bn);
-        std::vector<GroupedProblem> sorted;
-        sorted.reserve(probs.size());
+        auto tiles = [&](const GroupedProblem &g) { return ((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn); };
         int64_t t = 0;
-        for (int i : order) {
-            GroupedProblem g = probs[i];
-            g.tile_start = t;
-            t += ((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn);
-            sorted.push_back(g);
-        }
+        for (const GroupedProblem &g : probs) t += tiles(g);
         p->total_tiles[cfg] = t;
-        if (sorted.empty()) continue;
-        // descriptors, then their first tile indices (the kernels' search array)
-        std::vector<int64_t> starts;
-        for (const GroupedProblem &g : sorted) starts.push_back(g.tile_start);
-        // and the owner of every tile (direct-LDS kernels)
-        std::vector<int> owner;
-        if (p->dl >= 0) owner.reserve((size_t)t);
-        for (size_t i = 0; p->dl >= 0 && i < sorted.size(); ++i)
-            owner.insert(owner.end(), (size_t)((i + 1 < sorted.size() ? starts[i + 1] : t) - starts[i]), (int)i);
-        const size_t dbytes = sorted.size() * sizeof(GroupedProblem), sbytes = starts.size() * sizeof(int64_t);
-        const size_t obytes = owner.size() * sizeof(int);
-        hipError_t e = dev_alloc(reinterpret_cast<void **>(&p->dev[cfg]), dbytes + sbytes + obytes);
+        if (n == 0) continue;
+        image.resize(dbytes + sbytes + (p->dl >= 0 ? (size_t)t * sizeof(int) : 0));
+        GroupedProblem *sorted = reinterpret_cast<GroupedProblem *>(image.data());
+        int64_t *starts = reinterpret_cast<int64_t *>(image.data() + dbytes);
+        int *owner = reinterpret_cast<int *>(image.data() + dbytes + sbytes);
+        int64_t start = 0;
+        for (size_t i = 0; i < n; ++i) {
+            sorted[i] = probs[order[i]];
+            sorted[i].tile_start = starts[i] = start;
+            start += tiles(sorted[i]);
+            if (p->dl >= 0) std::fill(owner + starts[i], owner + start, (int)i);
+        }
+        hipError_t e = dev_alloc(reinterpret_cast<void **>(&p->dev[cfg]), image.size());
         if (e != hipSuccess) {
             (void)hipGetLastError();
             set_error("grouped dgemm: descriptor allocation failed (%s)", hipGetErrorString(e));
             rc = COSMA_AMD_ERR_ALLOC;
             break;
         }
-        e = hipMemcpy(p->dev[cfg], sorted.data(), dbytes, hipMemcpyHostToDevice);
-        if (e == hipSuccess)
-            e = hipMemcpy(reinterpret_cast<char *>(p->dev[cfg]) + dbytes, starts.data(), sbytes, hipMemcpyHostToDevice);
-        if (e == hipSuccess && obytes > 0)
-            e = hipMemcpy(reinterpret_cast<char *>(p->dev[cfg]) + dbytes + sbytes, owner.data(), obytes, hipMemcpyHostToDevice);
+        e = hipMemcpy(p->dev[cfg], image.data(), image.size(), hipMemcpyHostToDevice);
         if (e != hipSuccess) {
             set_error("grouped dgemm: descriptor upload failed (%s)", hipGetErrorString(e));
             rc = COSMA_AMD_ERR_HIP;
